@@ -50,8 +50,10 @@ extern "C" {
 #define WNW_ATTN_AUTO 0 /* fastest kernel that supports the arguments    */
 #define WNW_ATTN_MFMA 1 /* bf16/f16, head_dim 64/128, group <= 16         */
 #define WNW_ATTN_VALU 2 /* any dtype, head_dim 64/128/256, group <= 16    */
-#define WNW_ATTN_STREAM 3 /* bf16/f16, head_dim 64/128, group <= 8 (AUTO's
-                             choice there)                              */
+#define WNW_ATTN_STREAM 3 /* bf16/f16, head_dim 64/128, group <= 8 (by name;
+                             AUTO takes it for rows of up to 512 bytes: also
+                             groups of up to 16, 16-bit head_dim 256 and fp32
+                             head_dim 64/128)                           */
 
 /* Message describing the last failure on this thread ("" if none). */
 const char* wnw_last_error(void);
@@ -250,8 +252,8 @@ int wnw_decode_attn(const void* q, const void* k, const void* v,
  * cu_new = cu_old + arange(n_seg + 1) (the reference's cache.py:504), and
  * out is wnw_decode_attn over the len + 1 rows of every segment.  The
  * streaming kernel reads the new rows from new_k/new_v and writes them into
- * the pools itself (one launch); other kernels (fp32, head_dim 256, group
- * > 8) run wnw_append_inplace first.  total_rows (an estimate of
+ * the pools itself (one launch); where it does not apply (fp32 head_dim 256)
+ * wnw_append_inplace runs first.  total_rows (an estimate of
  * cu_old[n_seg] + n_seg) sizes the grid.
  * seg_cap[s] bounds len + 1 (WNW_DEVERR_CAPACITY otherwise; the row is then
  * attended but not stored).  cu_new must not alias cu_old.  new_k/new_v
@@ -332,8 +334,8 @@ int64_t wnw_decode_attn_score_workspace_bytes(int64_t n_seg, int64_t group,
  * sum is deterministic).  max_audio >= every audio_ends[b] - audio_starts[b]
  * (it sizes the grid); acc_len = entries of score_acc.  Audio ranges outside
  * a segment set WNW_DEVERR_BOUNDS and skip that segment.
- * When the streaming attention kernel runs (bf16/f16, head_dim 64/128,
- * group <= 8) and the workspace has room for the logits (see
+ * When the streaming attention kernel runs (rows of up to 512 bytes) and
+ * the workspace has room for the logits (see
  * wnw_decode_attn_score_workspace_bytes), the attention kernel keeps the
  * scaled logits of the scored rows and the scoring pass reads those instead
  * of K (4 bytes per row and head instead of 2 * head_dim).

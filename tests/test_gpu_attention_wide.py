@@ -1,0 +1,56 @@
+"""The streaming attention kernel's wide instances (q through registers):
+groups of 9 to 16 heads, 512-byte rows (fp32 head_dim 128, 16-bit head_dim
+256) and fp32 head_dim 64, against the float64 oracle at the edges of their
+16-row steps, wave ranges and segment table: fused append, dense operator
+and kept logits.  Tolerances as in test_gpu_attention.py (16-bit outputs
+2e-3 + 1e-2 |ref|, fp32 1e-4 + 1e-3 |ref|) and test_gpu_score.py (scores
+1e-6 + 1e-3 |ref|: sums of weights from 32-bit logits)."""
+import numpy as np
+import pytest
+
+from tests.helpers import allclose_report
+from tests.test_gpu_attention import _append_case, _check_append, _run_case, _tol
+
+pytestmark = pytest.mark.gpu
+
+WIDE = [("float32", 4, 64), ("float32", 16, 64), ("float32", 1, 128), ("float32", 9, 128), ("bfloat16", 9, 64),
+        ("float16", 16, 64), ("bfloat16", 13, 128), ("float16", 16, 128), ("bfloat16", 1, 256), ("float16", 8, 256),
+        ("bfloat16", 16, 256)]
+
+
+def _lens(n):
+    """n segments: empty, one-row, around one and two 16-row steps, long."""
+    edge = [0, 1, 15, 16, 17, 31, 32, 33, 48, 5000, 2, 64, 300]
+    rng = np.random.default_rng(n)
+    return (edge + [int(x) for x in rng.integers(0, 70, max(0, n - len(edge)))])[:n]
+
+
+@pytest.mark.parametrize("n", [13, 64, 65, 150])
+@pytest.mark.parametrize("dtype,G,D", WIDE)
+def test_append_and_dense(gpu, dtype, G, D, n):
+    """64 / 65 segments: the direct table and the table pass."""
+    _check_append(_append_case(gpu, _lens(n), G, D, dtype, seed=G + n), dtype)
+    for n_wg in (0, 1, 3):
+        got, ref = _run_case(gpu, _lens(n), G, D, dtype, n_wg=n_wg, seed=D + n)
+        ok, msg = allclose_report(got, ref, *_tol(dtype))
+        assert ok, msg
+
+
+@pytest.mark.parametrize("dtype,G,D", WIDE)
+def test_append_with_scores(gpu, dtype, G, D):
+    """The kept logits of the appended segments, scored by the logit pass."""
+    lens = [40, 300, 17, 1000, 64, 2, 513, 90]
+    r = _append_case(gpu, lens, G, D, dtype, seed=4, score=(4, [0, 1, 0, 1], [3, 0], [17, 2]))
+    _check_append(r, dtype)
+    acc, ref = r["extra"]
+    ok, msg = allclose_report(acc.cpu().numpy().astype(np.float64), ref, 1e-6, 1e-3)
+    assert ok, msg
+
+
+@pytest.mark.parametrize("dtype,G,D", [("float32", 4, 128), ("bfloat16", 16, 128), ("bfloat16", 5, 256)])
+def test_many_segments_per_wave(gpu, dtype, G, D):
+    """One workgroup over 300 segments: the walk changes windows, more new
+    rows end in a wave than it keeps until the end."""
+    rng = np.random.default_rng(5)
+    lens = [int(x) for x in rng.integers(0, 24, 300)]
+    _check_append(_append_case(gpu, lens, G, D, dtype, seed=8, rows_hint=64), dtype)

@@ -183,7 +183,7 @@ struct LogitScoreParams {
 
 static constexpr int kLogitThreads = 256;
 static constexpr int kLogitKv = 64;  // KV heads per sample this pass takes (a lane of wave 0 each)
-static constexpr int kLogitG = 8;    // query heads per KV head (the streaming kernel's limit)
+static constexpr int kLogitG = 8;    // query heads per KV head of a score slot
 
 // Latency, not bytes, bounds this pass (a few hundred KB per launch), so
 // its loads go out in two batches instead of a chain: wave 0 reads every
@@ -198,11 +198,14 @@ static constexpr int kLogitG = 8;    // query heads per KV head (the streaming k
 // delivers 14 in SGPRs at dispatch: the six tables of the first round trip
 // and the sizes their addresses need (hg = Hkv | G << 16, n_seg), so those
 // loads issue before any argument load returns.
+// KG: room for the query heads of a group (8, or 16 for wider groups, whose
+// first round trip loads twice the normalisers).
+template <int KG>
 __global__ __launch_bounds__(kLogitThreads) void logit_score_kernel(
     const int32_t* audio_s, const int32_t* audio_e, const int32_t* mask, const int32_t* cu, const int64_t* seg_base,
     const float* lse, int32_t hg, int32_t n_seg, LogitScoreParams p) {
   __shared__ int32_t seg_sh[kLogitKv];
-  __shared__ float m_sh[kLogitKv * kLogitG], inv_sh[kLogitKv * kLogitG];
+  __shared__ float m_sh[kLogitKv * KG], inv_sh[kLogitKv * KG];
   __shared__ int32_t n_sh;
   const int b = blockIdx.y;
   const int tid = threadIdx.x;
@@ -214,9 +217,9 @@ __global__ __launch_bounds__(kLogitThreads) void logit_score_kernel(
     const int32_t flag = mask[kv];
     const int64_t bv = seg_base ? seg_base[s] : 0;
     const int64_t c0 = cu[s], c1 = cu[s + 1];
-    float m[kLogitG], l[kLogitG];
+    float m[KG], l[KG];
 #pragma unroll
-    for (int g = 0; g < kLogitG; ++g) {
+    for (int g = 0; g < KG; ++g) {
       const int64_t e = ((int64_t)s * G + min(g, G - 1)) * 2;
       m[g] = lse[e];
       l[g] = lse[e + 1];
@@ -232,9 +235,9 @@ __global__ __launch_bounds__(kLogitThreads) void logit_score_kernel(
       const int pos = __popcll(bal & ((1ull << tid) - 1ull));
       seg_sh[pos] = s;
 #pragma unroll
-      for (int g = 0; g < kLogitG; ++g) {
-        m_sh[pos * kLogitG + g] = m[g];
-        inv_sh[pos * kLogitG + g] = 1.f / l[g];
+      for (int g = 0; g < KG; ++g) {
+        m_sh[pos * KG + g] = m[g];
+        inv_sh[pos * KG + g] = 1.f / l[g];
       }
     }
     if (tid == 0) n_sh = __popcll(bal);
@@ -274,7 +277,7 @@ __global__ __launch_bounds__(kLogitThreads) void logit_score_kernel(
       if (t0 + u < nt) {
         // v_exp_f32 directly: arguments are <= 0 (m is the maximum) and
         // weights below 2^-126 (flushed to zero) are negligible
-        sc += __builtin_amdgcn_exp2f(x[u] - m_sh[i * kLogitG + g]) * inv_sh[i * kLogitG + g];
+        sc += __builtin_amdgcn_exp2f(x[u] - m_sh[i * KG + g]) * inv_sh[i * KG + g];
         if (g == G - 1) {
           total += sc;
           sc = 0.f;
@@ -530,7 +533,7 @@ static int decode_attn_score_impl(const void* q, const void* k, const void* v, c
   lg.audio_e = audio_ends;
   lg.max_audio = max_audio;
   lg.hkv = (int32_t)num_kv_heads;
-  const bool room = max_audio > 0 && num_kv_heads <= kLogitKv && group <= kLogitG &&
+  const bool room = max_audio > 0 && num_kv_heads <= kLogitKv && group <= kMaxHeads &&
                     workspace_bytes >= xoff + n_seg * group * max_audio * 4;
   int kept = 0;
   int rc = decode_attn_impl(q, k, v, cu_k, seg_base, n_seg, group, head_dim, total_rows, kv_rows, scale,
@@ -547,10 +550,11 @@ static int decode_attn_score_impl(const void* q, const void* k, const void* v, c
     lp.kv_rows = kv_rows;
     lp.acc_len = acc_len;
     lp.max_audio = max_audio;
-    const int32_t hg = (int32_t)num_kv_heads | ((int32_t)group << 16);  // room: Hkv <= 64, G <= 8
+    const int32_t hg = (int32_t)num_kv_heads | ((int32_t)group << 16);  // room: Hkv <= 64, G <= 16
     const dim3 grid((unsigned)((max_audio + kLogitThreads - 1) / kLogitThreads), (unsigned)(n_seg / num_kv_heads));
-    hipLaunchKernelGGL(logit_score_kernel, grid, dim3(kLogitThreads), 0, (hipStream_t)stream, audio_starts,
-                       audio_ends, ca_kv_mask, cu_scored, seg_base, (const float*)lse, hg, (int32_t)n_seg, lp);
+    hipLaunchKernelGGL(group <= kLogitG ? logit_score_kernel<kLogitG> : logit_score_kernel<kMaxHeads>, grid,
+                       dim3(kLogitThreads), 0, (hipStream_t)stream, audio_starts, audio_ends, ca_kv_mask, cu_scored,
+                       seg_base, (const float*)lse, hg, (int32_t)n_seg, lp);
     WNW_CHECK_HIP(hipGetLastError(), "logit score launch");
     return WNW_OK;
   }
@@ -648,8 +652,8 @@ extern "C" int wnw_score_kept_logits(const int32_t* kv_mask, const float* slot, 
   lp.max_audio = max_audio;
   const int32_t hg = (int32_t)num_kv_heads | ((int32_t)group << 16);
   const dim3 grid((unsigned)((max_audio + kLogitThreads - 1) / kLogitThreads), (unsigned)(n_seg / num_kv_heads));
-  hipLaunchKernelGGL(logit_score_kernel, grid, dim3(kLogitThreads), 0, (hipStream_t)stream, audio_starts, audio_ends,
-                     kv_mask, cu, seg_base, slot, hg, (int32_t)n_seg, lp);
+  hipLaunchKernelGGL(logit_score_kernel<kLogitG>, grid, dim3(kLogitThreads), 0, (hipStream_t)stream, audio_starts,
+                     audio_ends, kv_mask, cu, seg_base, slot, hg, (int32_t)n_seg, lp);
   WNW_CHECK_HIP(hipGetLastError(), "logit score launch");
   return WNW_OK;
 }
@@ -774,6 +778,6 @@ extern "C" int wnw_fused_score_accumulate(const void* q, const void* k, const in
 namespace wnw {
 void touch_score_kernels() {
   hipFuncAttributes a;
-  (void)hipFuncGetAttributes(&a, (const void*)&logit_score_kernel);
+  (void)hipFuncGetAttributes(&a, (const void*)&logit_score_kernel<kLogitG>);
 }
 }  // namespace wnw
