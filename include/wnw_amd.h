@@ -204,8 +204,8 @@ int wnw_compact_segments(const void* src_k, const void* src_v, void* dst_k,
  * arrival counters; it must be cleared once with wnw_workspace_init before
  * its first use and may then be reused by any number of launches on one
  * stream (every launch leaves the counters at zero).  The counters occupy the
- * first 4 * n_seg bytes (rounded up to 256) and the partials follow them, so
- * a launch with another n_seg turns partial bytes into counters and the
+ * front, as many bytes as n_seg asks for, and the partials follow them, so a
+ * launch with another n_seg turns partial bytes into counters and the
  * reverse: clear the workspace again whenever n_seg changes.
  */
 int64_t wnw_decode_attn_workspace_bytes(int64_t n_seg, int64_t group,

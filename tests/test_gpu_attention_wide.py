@@ -54,3 +54,17 @@ def test_many_segments_per_wave(gpu, dtype, G, D):
     rng = np.random.default_rng(5)
     lens = [int(x) for x in rng.integers(0, 24, 300)]
     _check_append(_append_case(gpu, lens, G, D, dtype, seed=8, rows_hint=64), dtype)
+
+
+@pytest.mark.parametrize("dtype,G,D", [("bfloat16", 4, 128), ("float16", 16, 128), ("bfloat16", 7, 64),
+                                       ("float32", 2, 128)])
+@pytest.mark.parametrize("n_wg", [97, 256, 1100])
+def test_two_level_merge(gpu, dtype, G, D, n_wg):
+    """Segments of more than 32 pieces (merged block by block) side by side,
+    with one-row and empty segments between, at piece counts around whole
+    blocks of 16; twice on one workspace, whose counters must be left at zero."""
+    lens = [9000, 1, 4096, 0, 2, 4096, 5000, 1, 1, 1, 700]
+    for seed in (1, 2):
+        got, ref = _run_case(gpu, lens, G, D, dtype, n_wg=n_wg, seed=seed)
+        ok, msg = allclose_report(got, ref, *_tol(dtype))
+        assert ok, msg

@@ -12,6 +12,10 @@ static constexpr int kSplitWaves = 4;   // waves a workgroup's row range is cut 
 static constexpr int kPrevLogits = 16;  // pairs per sample the deferred form takes (<= 8 KV heads)
 static constexpr float kLog2e = 1.4426950408889634f;
 
+static constexpr int kPiecesPerBlock = 16;
+// Block partials of a launch of n_wg workgroups (two per 16 workgroups).
+constexpr int64_t attn_blocks(int64_t n_wg) { return 2 * (n_wg / kPiecesPerBlock + 1); }
+
 struct AttnParams {
   const void* q;        // [n_seg, G, D]
   const void* k;        // [phys_rows, D]
@@ -62,6 +66,12 @@ struct AttnParams {
   int64_t pv_acc_len;
   int32_t pv_nblk;  // 256-token blocks per sample
   int32_t pv_slices;  // samples x pv_nblk (<= the grid)
+  // two-level merge of long segments (streaming kernel, BLK instances; last, so that the
+  // fields every launch reads keep their cache lines): block partials and
+  // their arrival counters, attn_blocks(grid) of each
+  float* blk_acc;
+  float* blk_ml;
+  int32_t* blk_counters;
 };
 
 // Launches kernel WNW_ATTN_{MFMA,VALU,STREAM} for element type T.

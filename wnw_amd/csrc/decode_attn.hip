@@ -37,26 +37,33 @@ static DeviceInfo& device_info() {
 
 struct WsLayout {
   int64_t counters, ml, acc, total;
+  int64_t blk_counters, blk_ml, blk_acc;
   int64_t slots;
 };
 
-// Arrival counters for cap_seg segments first, then the (m, l) pairs and
-// the accumulators of `slots` partial slots.
-static WsLayout make_layout(int64_t cap_seg, int64_t slots, int64_t G, int64_t D) {
+// Arrival counters of cap_seg segments and `blocks` block partials first
+// (their place depends on cap_seg alone: a launch with another group or
+// head_dim finds them cleared), then the (m, l) pairs and the accumulators of
+// `slots` partial slots and of the block partials.
+static WsLayout make_layout(int64_t cap_seg, int64_t slots, int64_t G, int64_t D, int64_t blocks) {
   WsLayout L;
   L.slots = slots;
   auto up = [](int64_t x) { return (x + 255) / 256 * 256; };
   L.counters = 0;
-  L.ml = up(cap_seg * 4);
+  L.blk_counters = cap_seg * 4;
+  L.ml = up((cap_seg + blocks) * 4);
   L.acc = L.ml + up(L.slots * G * 2 * 4);
-  L.total = L.acc + up(L.slots * G * D * 4);
+  L.blk_ml = L.acc + up(L.slots * G * D * 4);
+  L.blk_acc = L.blk_ml + up(blocks * G * 2 * 4);
+  L.total = L.blk_acc + up(blocks * G * D * 4);
   return L;
 }
 
 // Caller-owned workspace: sized before the grid is known, so for the
 // largest grid a launch may use.
 static WsLayout ws_layout(int64_t n_seg, int64_t G, int64_t D) {
-  return make_layout(n_seg, device_info().max_wg + n_seg, G, D);
+  const int64_t wg = device_info().max_wg;
+  return make_layout(n_seg, wg + n_seg, G, D, attn_blocks(wg));
 }
 
 // ---------------------------------------------------------------------------
@@ -70,7 +77,13 @@ static WsLayout ws_layout(int64_t n_seg, int64_t G, int64_t D) {
 // calls with different n_seg never turn partial bytes into counters; every
 // launch leaves the counters of its segments at zero, the others are never
 // touched, and the array is zero at load (cleared again on first use).
-static constexpr int64_t kNoAllocBytes = WNW_NOALLOC_SCRATCH_BYTES;
+// WNW_NOALLOC_SCRATCH_BYTES bound a call's partials and segment counters; the
+// block partials (grids of up to kNoAllocWgs, two workgroups per CU) have
+// room of their own.
+static constexpr int64_t kNoAllocWgs = 1024;
+static constexpr int64_t kNoAllocBlocks = attn_blocks(kNoAllocWgs);
+static constexpr int64_t kNoAllocBytes =
+    WNW_NOALLOC_SCRATCH_BYTES + kNoAllocBlocks * (4 + kMaxGroup * (256 + 2) * 4) + 4 * 256;
 static __device__ __align__(256) uint8_t g_attn_scratch[kNoAllocBytes];
 
 struct ScratchSlot {
@@ -123,7 +136,7 @@ static int noalloc_scratch(hipStream_t st, void** out) {
     sl.ptr = p;
   }
   if (!sl.cleared) {
-    const int64_t n = (int64_t)WNW_NOALLOC_MAX_SEG;  // counters, 4 bytes each
+    const int64_t n = (int64_t)WNW_NOALLOC_MAX_SEG + kNoAllocBlocks;  // counters, 4 bytes each
     hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (uint32_t*)sl.ptr, n);
     WNW_CHECK_HIP(hipGetLastError(), "clearing the attention scratch counters");
     sl.cleared = true;
@@ -192,11 +205,13 @@ int decode_attn_impl(const void* q, const void* k, const void* v, const int32_t*
     // 128 elements and groups of up to 8, whatever the kernel launches
     const bool narrow = dtype != WNW_F32 && head_dim <= 128 && group <= kMaxGroupS;
     const int64_t P_lim = std::min<int64_t>((int64_t)di.cus * (narrow ? 1 : 2), std::max<int64_t>(1, (total_rows + 63) / 64));
-    L = make_layout(WNW_NOALLOC_MAX_SEG, std::max(P, P_lim) + n_seg, group, head_dim);
-    WNW_CHECK_ARG(L.total <= kNoAllocBytes,
+    P = std::min(P, kNoAllocWgs);
+    const WsLayout lim = make_layout(WNW_NOALLOC_MAX_SEG, std::max(P, P_lim) + n_seg, group, head_dim, 0);
+    WNW_CHECK_ARG(lim.total <= WNW_NOALLOC_SCRATCH_BYTES,
                   "this launch needs %lld bytes of split-K scratch; the no-alloc entry point holds %lld "
                   "(fewer segments or a smaller group / head_dim fit)",
-                  (long long)L.total, (long long)kNoAllocBytes);
+                  (long long)lim.total, (long long)WNW_NOALLOC_SCRATCH_BYTES);
+    L = make_layout(WNW_NOALLOC_MAX_SEG, std::max(P, P_lim) + n_seg, group, head_dim, kNoAllocBlocks);
     const int rc = noalloc_scratch((hipStream_t)stream, &workspace);
     if (rc != WNW_OK) return rc;
   } else {
@@ -216,6 +231,9 @@ int decode_attn_impl(const void* q, const void* k, const void* v, const int32_t*
   ap.lse = lse;
   ap.part_ml = (float*)((char*)workspace + L.ml);
   ap.part_acc = (float*)((char*)workspace + L.acc);
+  ap.blk_counters = (int32_t*)((char*)workspace + L.blk_counters);
+  ap.blk_ml = (float*)((char*)workspace + L.blk_ml);
+  ap.blk_acc = (float*)((char*)workspace + L.blk_acc);
   ap.err = device_error_word();
   ap.split_inv = ~0ull / (uint64_t)(P * kSplitWaves) + 1;  // ceil(2^64 / (P * kSplitWaves))
   ap.phys_rows = kv_rows;

@@ -526,20 +526,39 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 0xF) | ((N & 0x30) << 10));
 }
 
-// Last-arriver merge of the np partials of one segment (slots s0 ..
-// s0 + np - 1) into the output, by threads t = 0 .. nt - 1.  Every thread
-// owns 4 consecutive elements of one head and reads, for a chunk of partials
-// at a time, their (m, l) pairs and its accumulator quad: one memory round
-// trip per chunk, no LDS and no barriers.  The reads are buffer loads with
-// the sc1 policy (the agent-coherent form of a load on gfx950), one 16-byte
-// and one 8-byte load per partial at a scalar offset from the segment's
-// first slot.  Chunks are folded in slot order with the usual max
-// rescaling, so the result is deterministic.
-template <typename T>
+// Segments of more than kBlkMin pieces merge in two levels (streaming kernel):
+// the last arriver of each block of kBlk consecutive pieces folds the block
+// into one block partial, and the last of a segment's blocks folds those.
+// All but the last block's folding happens while other workgroups still
+// stream; one last arriver folding every piece chained a memory round trip per
+// 16 of them (one sample of 22,600 rows over 256 workgroups: 95 pieces).  Two round
+// trips (up to 32 pieces) cost less than the second hand-off.
+// Block j of a segment whose first piece is workgroup p_first's gets index
+// block_index(p_first / 16, j).  No two blocks of a launch share one: a
+// segment's blocks start 16 workgroups apart, so at most one in each bucket of
+// 16; and of two segments with a block start in one bucket the earlier one's
+// is not its first block (it has more than 32 pieces, the later segment
+// starts where it ends or after) and the later one's is its first.
+static constexpr int kBlk = 16;
+static constexpr int kBlkMin = 32;
+static_assert(kBlk == kPiecesPerBlock, "the workspace is sized for this block");
+__device__ __forceinline__ int block_index(int bucket, int j) { return 2 * (bucket + j) + (j > 0 ? 1 : 0); }
+
+// Merge of np partials of segment s (slots s0 .. s0 + np - 1) by threads
+// t = 0 .. nt - 1: into the output, or (BLK, with dst_acc) as one partial there.
+// Every thread owns 4 consecutive elements of one head and reads, for a
+// chunk of partials at a time, their (m, l) pairs and its accumulator quad:
+// one memory round trip per chunk, no LDS and no barriers.  The reads are
+// buffer loads with the sc1 policy (the agent-coherent form of a load on
+// gfx950), one 16-byte and one 8-byte load per partial at a scalar offset
+// from the first.  Chunks are folded in slot order with the usual max
+// rescaling, so the result is deterministic.  blocks (BLK): the partials are
+// a segment's block partials (block_index), the first at index s0.
+template <typename T, bool BLK>
 __device__ __forceinline__ void combine_pieces(const AttnParams& p, int D, int64_t s0, int np, int64_t s, int t,
-                                               int nt) {
-  // the segment and its slots are wave-uniform: scalar, so the buffer
-  // descriptors below live in SGPRs
+                                               int nt, bool blocks = false, float* dst_acc = nullptr,
+                                               float* dst_ml = nullptr) {
+  // wave-uniform values: scalar, so the buffer descriptors below live in SGPRs
   s0 = uni(s0);
   np = uni(np);
   s = uni(s);
@@ -550,10 +569,11 @@ __device__ __forceinline__ void combine_pieces(const AttnParams& p, int D, int64
   const int G = p.G;
   const int GD = G * D;
   const int GD4 = GD / 4;
-  const __amdgpu_buffer_rsrc_t ra =
-      __builtin_amdgcn_make_buffer_rsrc(p.part_acc + s0 * GD, 0, np * GD * 4, kRsrc3);
-  const __amdgpu_buffer_rsrc_t rm =
-      __builtin_amdgcn_make_buffer_rsrc(p.part_ml + s0 * G * 2, 0, np * G * 8, kRsrc3);
+  const int span = BLK && blocks ? 2 * np : np;
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+      (BLK && blocks ? p.blk_acc : p.part_acc) + s0 * GD, 0, span * GD * 4, kRsrc3);
+  const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(
+      (BLK && blocks ? p.blk_ml : p.part_ml) + s0 * G * 2, 0, span * G * 8, kRsrc3);
   for (int i4 = t; i4 < GD4; i4 += nt) {
     const int g = (4 * i4) / D;
     float M = kNegBig, L = 0.f;
@@ -566,9 +586,9 @@ __device__ __forceinline__ void combine_pieces(const AttnParams& p, int D, int64
         a[k] = f32x4{0.f, 0.f, 0.f, 0.f};
         ml[k] = u32x2{0u, 0u};
         if (q0 + k < np) {  // wave-uniform: no wait between the loads
-          a[k] = __builtin_bit_cast(f32x4,
-                                    __builtin_amdgcn_raw_buffer_load_b128(ra, i4 * 16, (q0 + k) * GD * 4, kSc1));
-          ml[k] = __builtin_amdgcn_raw_buffer_load_b64(rm, g * 8, (q0 + k) * G * 8, kSc1);
+          const int at = BLK && blocks ? block_index(0, q0 + k) : q0 + k;
+          a[k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, i4 * 16, at * GD * 4, kSc1));
+          ml[k] = __builtin_amdgcn_raw_buffer_load_b64(rm, g * 8, at * G * 8, kSc1);
         }
       }
       float Mc = M;
@@ -587,10 +607,17 @@ __device__ __forceinline__ void combine_pieces(const AttnParams& p, int D, int64
       }
       M = Mc;
     }
+    const bool lead = (4 * i4) % D == 0;
+    if (BLK && dst_acc) {
+      st_agent2(dst_acc + 4 * i4, A[0], A[1]);
+      st_agent2(dst_acc + 4 * i4 + 2, A[2], A[3]);
+      if (lead) st_agent2(dst_ml + g * 2, M, L);
+      continue;
+    }
     const float inv = 1.f / L;
     const float o4[4] = {A[0] * inv, A[1] * inv, A[2] * inv, A[3] * inv};
     store_quad<T>(p.out, s * GD + 4 * i4, o4);
-    if (p.lse && (4 * i4) % D == 0) {
+    if (p.lse && lead) {
       gptr_w<float>(p.lse)[(s * G + g) * 2] = M;
       gptr_w<float>(p.lse)[(s * G + g) * 2 + 1] = L;
     }
@@ -617,16 +644,6 @@ __device__ __forceinline__ bool arrive(const AttnParams& p, const SchedLds& sl, 
   return old == (int)(p_last - p_first);
 }
 
-// The merge of segment s from its np pieces, the first held by workgroup
-// p_first (by threads t = 0 .. nt - 1), and the reset of its counter for the
-// next launch.
-template <typename T>
-__device__ __forceinline__ void combine_from(const AttnParams& p, int D, int64_t p_first, int np, int s, int t,
-                                             int nt) {
-  combine_pieces<T>(p, D, p_first + s /* slot of the first piece */, np, s, t, nt);
-  if (t == 0) __hip_atomic_store(gptr_w<int32_t>(p.counters) + s, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // The last arriver of segment s merges every partial into the output (by
 // threads t = 0 .. nt - 1 of the workgroup) and resets the counter for the
 // next launch.  No LDS is used.
@@ -635,7 +652,8 @@ __device__ __forceinline__ void combine_segment(const AttnParams& p, int D, cons
                                                 int64_t seg_len, int s, int t, int nt) {
   int64_t p_first, p_last;
   piece_range(sl, seg_lo, seg_len, p_first, p_last);
-  combine_from<T>(p, D, p_first, (int)(p_last - p_first + 1), s, t, nt);
+  combine_pieces<T, false>(p, D, p_first + s /* slot of the first piece */, (int)(p_last - p_first + 1), s, t, nt);
+  if (t == 0) __hip_atomic_store(gptr_w<int32_t>(p.counters) + s, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Arrival of this workgroup's partial of segment s followed, on the last
@@ -1180,7 +1198,10 @@ struct SStep {
 // PV: score the previous launch's kept logits (deferred scoring; direct
 // table and fused append only), an instance of its own so that the other
 // launches carry none of its code or argument loads.
-template <typename T, int D, int NW, int QD, bool XL, bool APPEND, bool DIRECT, bool PV = false>
+// BLK: merge segments of more than kBlkMin pieces in two levels, an instance of
+// its own because that code costs every launch that never takes it ~0.25 us
+// (20.15 -> 20.4 us per fused launch at 64 segments of up to 7,564 rows).
+template <typename T, int D, int NW, int QD, bool XL, bool APPEND, bool DIRECT, bool PV, bool BLK>
 // The fields read first lead the argument list as scalars: the build asks
 // for 16 preloaded argument dwords (-amdgpu-kernarg-preload-count), of which
 // the hardware delivers 14 in SGPRs at dispatch (the other two user SGPRs
@@ -1965,13 +1986,22 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
   wait_vmem();
   __syncthreads();  // partials complete; the slots may be overwritten below
   // Both arrivals in one atomic instruction (lanes 0 and 1 of wave 0, one
-  // memory round trip); each segment whose last partial this is merges.
+  // memory round trip); each segment (or block of one) whose last partial
+  // this is merges.
   if (tid < 2) {
     const int32_t ps = sl.order_bad ? -1 : (tid ? ps1 : ps0);
+    const int32_t pn = tid ? pn1 : pn0, pf = (int32_t)(tid ? pf1 : pf0);
     bool f = false;
-    if (ps >= 0)
-      f = __hip_atomic_fetch_add(gptr_w<int32_t>(p.counters) + ps, 1, __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT) == (tid ? pn1 : pn0);
+    if (ps >= 0) {
+      int32_t last = pn;
+      WNW_GLOBAL int32_t* c = gptr_w<int32_t>(p.counters) + ps;
+      if (BLK && pn >= kBlkMin) {
+        const int32_t j = ((int32_t)blockIdx.x - pf) / kBlk;
+        last = min(kBlk - 1, pn - kBlk * j);
+        c = gptr_w<int32_t>(p.blk_counters) + block_index(pf / kBlk, j);
+      }
+      f = __hip_atomic_fetch_add(c, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == last;
+    }
     const uint64_t fl = __ballot(f);
     if (tid == 0) sl.is_last = (int)(fl & 3);
   }
@@ -1994,7 +2024,40 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
     const bool both = last == 3;
     const int nt = both ? NT / 2 : NT;
     const bool k = both ? tid >= NT / 2 : last == 2;  // uniform per wave
-    combine_from<T>(p, D, k ? pf1 : pf0, (k ? pn1 : pn0) + 1, k ? ps1 : ps0, both && k ? tid - NT / 2 : tid, nt);
+    const int t = both && k ? tid - NT / 2 : tid;
+    const int32_t ps = k ? ps1 : ps0, np = (k ? pn1 : pn0) + 1, pf = (int32_t)(k ? pf1 : pf0);
+    const bool blk = BLK && np > kBlkMin;
+    const int32_t j = blk ? ((int32_t)blockIdx.x - pf) / kBlk : 0;
+    const int32_t bi = blk ? block_index(pf / kBlk, j) : 0;
+    const int64_t slot = (int64_t)pf + kBlk * j + ps;
+    combine_pieces<T, BLK>(p, D, slot, blk ? min(kBlk, np - kBlk * j) : np, ps, t, nt, false,
+                           blk ? p.blk_acc + (int64_t)bi * GD : nullptr, BLK ? p.blk_ml + (int64_t)bi * G * 2 : nullptr);
+    if (t == 0)
+      __hip_atomic_store(BLK && blk ? gptr_w<int32_t>(p.blk_counters) + bi : gptr_w<int32_t>(p.counters) + ps, 0,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // the segments' block arrivals, and the merge of the blocks by the last
+    const int at = BLK ? last & ((pn0 >= kBlkMin ? 1 : 0) | (pn1 >= kBlkMin ? 2 : 0)) : 0;  // workgroup-uniform
+    if (BLK && at) {
+      wait_vmem();
+      __syncthreads();  // block partials complete, is_last read by everyone
+      if (tid < 2) {
+        const int32_t s2 = tid ? ps1 : ps0, nb = (tid ? pn1 : pn0) / kBlk;  // blocks - 1
+        const bool f = ((at >> tid) & 1) && __hip_atomic_fetch_add(gptr_w<int32_t>(p.counters) + s2, 1, __ATOMIC_RELAXED,
+                                                                   __HIP_MEMORY_SCOPE_AGENT) == nb;
+        const uint64_t fl = __ballot(f);
+        if (tid == 0) sl.is_last = (int)(fl & 3);
+      }
+      __syncthreads();
+      const int last2 = uni(sl.is_last);
+#pragma unroll 1
+      for (int i = 0; i < 2; ++i) {
+        if (!((last2 >> i) & 1)) continue;  // workgroup-uniform
+        const int32_t s2 = i ? ps1 : ps0, b0 = block_index((int32_t)(i ? pf1 : pf0) / kBlk, 0);
+        combine_pieces<T, BLK>(p, D, b0, (i ? pn1 : pn0) / kBlk + 1, s2, tid, NT, true);
+        if (tid == 0)
+          __hip_atomic_store(gptr_w<int32_t>(p.counters) + s2, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
   }
   if (APPEND) {
     // (direct table) workgroup 0's post-append offsets, last, so no wait of
@@ -2158,7 +2221,7 @@ static hipError_t set_lds_limit_once(std::vector<signed char>& done, std::mutex&
 // Streaming kernel launch: QD = q loads per step, dynamic LDS as sized by
 // stream_lds_bytes (above 64 KB, so the limit is raised once per instance
 // and device).
-template <typename T, int D, int QD, bool XL, bool APPEND, bool DIRECT, bool PV = false>
+template <typename T, int D, int QD, bool XL, bool APPEND, bool DIRECT, bool PV, bool BLK>
 static hipError_t launch_stream_k(const AttnParams& ap, int64_t n_wg, hipStream_t st) {
   constexpr int side = stream_side_rows(XL, DIRECT);
   constexpr int RB = D * (int)sizeof(T);
@@ -2168,25 +2231,41 @@ static hipError_t launch_stream_k(const AttnParams& ap, int64_t n_wg, hipStream_
   static std::mutex mu;
   static std::vector<signed char> done;
   const hipError_t attr_err =
-      set_lds_limit_once(done, mu, (const void*)&attn_stream_kernel<T, D, kNW, QD, XL, APPEND, DIRECT, PV>,
+      set_lds_limit_once(done, mu, (const void*)&attn_stream_kernel<T, D, kNW, QD, XL, APPEND, DIRECT, PV, BLK>,
                          lds_max);
   if (attr_err != hipSuccess) return attr_err;
-  hipLaunchKernelGGL((attn_stream_kernel<T, D, kNW, QD, XL, APPEND, DIRECT, PV>), dim3((unsigned)n_wg), dim3(kNW * 64), lds,
-                     st, ap.cu, ap.base, ap.cap, ap.q, ap.k, ap.v, ap.n_seg,
+  hipLaunchKernelGGL((attn_stream_kernel<T, D, kNW, QD, XL, APPEND, DIRECT, PV, BLK>), dim3((unsigned)n_wg),
+                     dim3(kNW * 64), lds, st, ap.cu, ap.base, ap.cap, ap.q, ap.k, ap.v, ap.n_seg,
                      (int32_t)((uint32_t)ap.G | ((uint32_t)n_wg << 8)), ap.split_inv, ap);
   return hipGetLastError();
 }
 
 // Up to 64 segments the table is read by every wave directly (one lane per
-// segment); more take the workgroup scheduling pass.
+// segment); more take the workgroup scheduling pass.  A launch of at least
+// kBlkWgs workgroups, eight or more of them per segment, may well hold segments of
+// more than kBlkMin pieces and takes the instance that merges those in two
+// levels: 8 segments, two of 22,628 rows (95 pieces each) 24.9 -> 20.2 us; 16
+// segments, fp16, 16 heads, up to 86 pieces 32.4 -> 26.9 us.  With more segments or
+// fewer workgroups the long ones rarely pass 32 pieces and the instance's
+// cost is not earned (64 segments, 16 of ~7,300 ragged rows: 31.5 -> 32.2 us; 41
+// workgroups, 8 segments: 10.0 -> 10.4 us).  With q in registers there is
+// the one direct instance (such launches' accumulators are wide and the
+// chain of round trips long).
+static constexpr int kBlkWgs = 128;
 template <typename T, int D, int QD, bool XL, bool APPEND>
 static hipError_t launch_stream(const AttnParams& ap, int64_t n_wg, hipStream_t st) {
+  [[maybe_unused]] const bool blk = n_wg >= kBlkWgs && n_wg >= 8 * (int64_t)ap.n_seg;
   if constexpr (APPEND && QD > 0) {
-    if (ap.pv_xlog)  // the host allows it with the direct table only
-      return ap.n_seg <= 64 ? launch_stream_k<T, D, QD, XL, APPEND, true, true>(ap, n_wg, st) : hipErrorInvalidValue;
+    if (ap.pv_xlog) {  // the host allows it with the direct table only
+      if (ap.n_seg > 64) return hipErrorInvalidValue;
+      return blk ? launch_stream_k<T, D, QD, XL, APPEND, true, true, true>(ap, n_wg, st)
+                 : launch_stream_k<T, D, QD, XL, APPEND, true, true, false>(ap, n_wg, st);
+    }
   }
-  return ap.n_seg <= 64 ? launch_stream_k<T, D, QD, XL, APPEND, true>(ap, n_wg, st)
-                        : launch_stream_k<T, D, QD, XL, APPEND, false>(ap, n_wg, st);
+  if (ap.n_seg > 64) return launch_stream_k<T, D, QD, XL, APPEND, false, false, false>(ap, n_wg, st);
+  if constexpr (QD > 0)
+    if (!blk) return launch_stream_k<T, D, QD, XL, APPEND, true, false, false>(ap, n_wg, st);
+  return launch_stream_k<T, D, QD, XL, APPEND, true, false, true>(ap, n_wg, st);
 }
 
 template <typename T, int D, int QD>
