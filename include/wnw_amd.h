@@ -379,7 +379,7 @@ int64_t wnw_fused_score_workspace_bytes(int64_t n_samples, int64_t n_heads);
  * scale * q . K (the reference uses scale = head_dim^-0.5), summed over the
  * heads, is added at the audio rows [audio_starts[i], audio_ends[i])
  * (relative to seg_starts[i]) to accumulator[accum_offsets[i] + j].
- * Two launches: partial statistics over 32 row slices per item, then the
+ * Two launches: partial statistics over row slices of each item, then the
  * scoring pass over the audio rows.  k_rows = rows of k (bounds).
  */
 int wnw_fused_score_accumulate(const void* q, const void* k,

@@ -13,16 +13,20 @@
 //     audio rows of the flagged segments remains;
 //   * or a statistics pass (fused_score_accumulate, which scores a subset of
 //     a group's heads with its own scale): the rows of each segment are cut
-//     into kStatChunks slices whose partial (max, sum) pairs the scoring
-//     pass merges.
+//     into slices whose partial (max, sum) pairs the scoring pass merges.
 // The scoring pass gives one (sample, row range) to one workgroup, which
 // sums over heads (and over flagged KV heads) in registers and adds to the
 // accumulator once per token: no atomics, deterministic results.
 //
-// Row dot products: a row of D elements is read by D / EPC lanes, 16 bytes
-// each (one 64-byte-aligned run per lane group), and reduced across those
-// lanes with a butterfly; q lives in LDS as fp32.
+// Row dot products are 16 x 16 matrix instructions (rows x heads) in the
+// fused_score_accumulate passes.  In attn_score_kernel (kept for callers
+// without room for the logits) a row of D elements is read by D / EPC lanes,
+// 16 bytes each, and reduced across those lanes with a butterfly; q lives in
+// LDS as fp32.
 #include <math.h>
+
+#include <algorithm>
+#include <type_traits>
 
 #include "wnw_common.h"
 
@@ -33,7 +37,6 @@ static constexpr int kScoreThreads = 256;
 // (few samples or short audio).
 static constexpr int kIters = 16;
 static constexpr int kItersSmall = 4;
-static constexpr int kStatChunks = 32;    // row slices per segment in the statistics pass
 static constexpr int kMaxHeads = 16;
 static constexpr float kLog2eS = 1.4426950408889634f;
 static constexpr float kNegBigS = -1e30f;
@@ -304,12 +307,32 @@ struct SegScoreParams {
   const int32_t* audio_e;
   const int32_t* acc_off;  // [S + 1]
   float* acc;
-  float* part;             // [S, kStatChunks, nh, 2]
+  float* part;             // [S, slices, nh, 2] (max, sum) in the log2 domain
   int32_t* err;
   int64_t k_rows, acc_len;
   int32_t S, nh;
   float scale_log2;
 };
+
+// 16 rows x 16 heads of q . K: A = the rows' 16-byte chunks, B = q's, lane
+// (lq, lc) = (lane / 16, lane % 16) holding chunk 4 c + lq of row / head lc;
+// the sum's lane holds rows 4 lq + i of head lc.  16-bit products are exact in
+// the 32-bit sums, and fp32 runs on 32-bit matrix operands.
+template <typename T>
+__device__ __forceinline__ f32x4 dot_chunk(const u32x4& a, const u32x4& b, f32x4 c) {
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[j]), __uint_as_float(b[j]), c, 0, 0, 0);
+    return c;
+  } else if constexpr (std::is_same<T, bf16_t>::value) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+                                                   0, 0);
+  } else {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
+                                                  0);
+  }
+}
 
 __device__ __forceinline__ void merge_ml(float& m, float& l, float m2, float l2) {
   const float mn = fmaxf(m, m2);
@@ -317,149 +340,199 @@ __device__ __forceinline__ void merge_ml(float& m, float& l, float m2, float l2)
   m = mn;
 }
 
-template <typename T, int D>
-__global__ __launch_bounds__(kScoreThreads) void seg_stats_kernel(SegScoreParams p) {
-  constexpr int EPC = RowGeom<T>::EPC;
-  constexpr int LPR = D / EPC;
-  constexpr int RPI = kScoreThreads / LPR;
-  __shared__ float qf[kMaxHeads * D];
-  __shared__ float red[kScoreThreads / 64][kMaxHeads][2];
-  const int s = blockIdx.y, c = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int sub = tid % LPR, rl = tid / LPR;
-  const int64_t r0 = p.seg_s[s], r1 = p.seg_e[s];
-  const bool ok = r0 >= 0 && r1 >= r0 && r1 <= p.k_rows;
-  if (!ok && tid == 0 && c == 0) raise_device_error(p.err, WNW_DEVERR_BOUNDS);
-  const int64_t len = ok ? r1 - r0 : 0;
-  const int64_t c0 = r0 + len * c / kStatChunks, c1 = r0 + len * (c + 1) / kStatChunks;
-  stage_q<T>(qf, (const T*)p.q + (int64_t)s * p.nh * D, p.nh, D);
-  __syncthreads();
-  float m[kMaxHeads], l[kMaxHeads];
+// The 16 bytes at p, read whole where q is 16-byte aligned, else by element.
+template <typename T>
+__device__ __forceinline__ u32x4 load_chunk(const T* p, bool aligned) {
+  if (aligned) return *gptr<u32x4>(p);
+  constexpr int N = 16 / (int)sizeof(T);
+  u32x4 r = u32x4{0, 0, 0, 0};
 #pragma unroll
-  for (int h = 0; h < kMaxHeads; ++h) {
-    m[h] = kNegBigS;
-    l[h] = 0.f;
+  for (int i = 0; i < N; ++i) {
+    if constexpr (sizeof(T) == 4)
+      r[i] = gptr<uint32_t>(p)[i];
+    else
+      r[i / 2] |= (uint32_t)gptr<uint16_t>(p)[i] << (16 * (i & 1));
   }
-  const T* kp = (const T*)p.k;
-  for (int64_t row0 = c0; row0 < c1; row0 += RPI) {
-    const int64_t row = row0 + rl;
-    const bool valid = row < c1;
-    u32x4 wv = *(const u32x4*)(kp + (valid ? row : c0) * D + sub * EPC);
-    float kf[EPC];
-    chunk_to_f32<T>(wv, kf);
-#pragma unroll
-    for (int h = 0; h < kMaxHeads; ++h) {
-      if (h < p.nh) {
-        float d = 0.f;
-#pragma unroll
-        for (int i = 0; i < EPC; ++i) d += qf[h * D + sub * EPC + i] * kf[i];
-        d = group_sum<LPR>(d);
-        if (valid) merge_ml(m[h], l[h], d * p.scale_log2, 1.f);
-      }
-    }
-  }
-  // merge the row groups of the wave (one representative lane per group),
-  // then the waves through LDS
-#pragma unroll
-  for (int h = 0; h < kMaxHeads; ++h) {
-    if (h < p.nh) {
-      for (int o = LPR; o < 64; o <<= 1) {
-        const float m2 = __shfl_xor(m[h], o), l2 = __shfl_xor(l[h], o);
-        merge_ml(m[h], l[h], m2, l2);
-      }
-      if (lane == 0) {
-        red[w][h][0] = m[h];
-        red[w][h][1] = l[h];
-      }
-    }
-  }
-  __syncthreads();
-  if (tid < p.nh) {
-    float M = kNegBigS, Lsum = 0.f;
-    for (int ww = 0; ww < kScoreThreads / 64; ++ww) merge_ml(M, Lsum, red[ww][tid][0], red[ww][tid][1]);
-    float* out = p.part + (((int64_t)s * kStatChunks + c) * p.nh + tid) * 2;
-    out[0] = M;
-    out[1] = Lsum;
-  }
+  return r;
 }
 
-template <typename T, int D, int IT>
+// Slices per item: enough workgroups for two per CU of a 256-CU device, each
+// still with a few 16-row tiles (8 items of 7,564 rows: 64 slices of 118 rows).
+static int64_t score_slices(int64_t n_samples) {
+  return std::min<int64_t>(128, std::max<int64_t>(8, (512 + n_samples - 1) / std::max<int64_t>(n_samples, 1)));
+}
+
+// Both passes, one workgroup per slice of an item's rows (SCORE 0: the
+// slice's partial softmax statistics of every head; SCORE 1: every head's
+// statistics merged, then each audio row's weights summed over the heads and
+// added to its accumulator entry).  The passes cut the rows alike, so the
+// second one's K comes from the L2 of the XCD that the first one's
+// workgroups filled.  Bound by the K stream and by two launches' fixed round
+// trips; a row dot by 16-lane butterflies (six lane exchanges per row and
+// head) had bound it before: 25.1 + 10.4 us for 8 items of 7,564 rows, 4 heads,
+// bf16 D = 128 (15.5 MB), now 6.4 + 7.4 us.
+template <typename T, int D, bool SCORE>
 __global__ __launch_bounds__(kScoreThreads) void seg_score_kernel(SegScoreParams p) {
   constexpr int EPC = RowGeom<T>::EPC;
-  constexpr int LPR = D / EPC;
-  constexpr int RPI = kScoreThreads / LPR;
-  __shared__ float qf[kMaxHeads * D];
+  constexpr int NC = D / EPC / 4;           // chunks of a row per lane
+  constexpr int U = NC >= 8 ? 1 : 8 / NC;   // tiles whose loads are in flight per wave
+  constexpr int NW = kScoreThreads / 64;
   __shared__ float stat[kMaxHeads][2];
-  const int s = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int sub = tid % LPR, rl = tid / LPR;
-  const int64_t r0 = p.seg_s[s], r1 = p.seg_e[s];
-  const int a0 = p.audio_s[s], a1 = p.audio_e[s];
-  const int n_audio = a1 - a0;
-  const int j0 = blockIdx.x * RPI * IT;
-  if (j0 >= n_audio) return;
-  const int64_t off = p.acc_off[s];
-  if (r0 < 0 || r1 < r0 || r1 > p.k_rows || a0 < 0 || r0 + a1 > r1 || off < 0 || off + n_audio > p.acc_len) {
-    if (tid == 0) raise_device_error(p.err, WNW_DEVERR_BOUNDS);
-    return;
-  }
-  stage_q<T>(qf, (const T*)p.q + (int64_t)s * p.nh * D, p.nh, D);
-  // merge the statistics slices: wave w takes heads w, w + 4, ...
-  for (int h = w; h < p.nh; h += kScoreThreads / 64) {
-    const float* pp = p.part + ((int64_t)s * kStatChunks * p.nh + h) * 2;
-    const float mq = lane < kStatChunks ? pp[(int64_t)lane * p.nh * 2] : kNegBigS;
-    const float lq = lane < kStatChunks ? pp[(int64_t)lane * p.nh * 2 + 1] : 0.f;
-    const float M = wave_max(mq);
-    const float Lsum = wave_sum(lq * exp2f(mq - M));
-    if (lane == 0) {
-      stat[h][0] = M;
-      stat[h][1] = 1.f / Lsum;
+  __shared__ float red[SCORE ? 1 : NW][kMaxHeads][2];
+  const int s = blockIdx.y, c = blockIdx.x, C = gridDim.x;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lq = lane >> 4, lc = lane & 15;
+  const int nh = p.nh;
+  const int64_t r0 = gptr<int32_t>(p.seg_s)[s], r1 = gptr<int32_t>(p.seg_e)[s];
+  int64_t c0, c1;       // this workgroup's rows of k
+  int64_t off = 0, a_row = 0;
+  if constexpr (SCORE) {
+    const int a0 = gptr<int32_t>(p.audio_s)[s], a1 = gptr<int32_t>(p.audio_e)[s];
+    const int n_audio = a1 - a0;
+    off = gptr<int32_t>(p.acc_off)[s];
+    if (n_audio <= 0) return;
+    if (r0 < 0 || r1 < r0 || r1 > p.k_rows || a0 < 0 || r0 + a1 > r1 || off < 0 || off + n_audio > p.acc_len) {
+      if (tid == 0) raise_device_error(p.err, WNW_DEVERR_BOUNDS);
+      return;
     }
+    a_row = r0 + a0;
+    c0 = max(r0 + (r1 - r0) * c / C, a_row);
+    c1 = min(r0 + (r1 - r0) * (c + 1) / C, r0 + a1);
+    if (c0 >= c1) return;  // workgroup-uniform
+  } else {
+    const bool ok = r0 >= 0 && r1 >= r0 && r1 <= p.k_rows;
+    if (!ok && tid == 0 && c == 0) raise_device_error(p.err, WNW_DEVERR_BOUNDS);
+    const int64_t len = ok ? r1 - r0 : 0;
+    c0 = r0 + len * c / C;
+    c1 = r0 + len * (c + 1) / C;
   }
-  __syncthreads();
+  const int ntiles = (int)((c1 - c0 + 15) / 16);
   const T* kp = (const T*)p.k;
-  for (int it = 0; it < IT; ++it) {
-    const int j = j0 + it * RPI + rl;
-    const bool valid = j < n_audio;
-    const int64_t row = r0 + a0 + (valid ? j : 0);
-    u32x4 wv = *(const u32x4*)(kp + row * D + sub * EPC);
-    float kf[EPC];
-    chunk_to_f32<T>(wv, kf);
-    float sc = 0.f;
-    for (int h = 0; h < p.nh; ++h) {
-      float d = 0.f;
+  u32x4 kb[U][NC];
+  // tile t0 + NW u of the slice into kb[u]; rows past the slice repeat its last
+  auto load = [&](int t0) {
 #pragma unroll
-      for (int i = 0; i < EPC; ++i) d += qf[h * D + sub * EPC + i] * kf[i];
-      d = group_sum<LPR>(d);
-      sc += exp2f(d * p.scale_log2 - stat[h][0]) * stat[h][1];
+    for (int u = 0; u < U; ++u) {
+      const int64_t row = min(c0 + 16 * (int64_t)(t0 + NW * u) + lc, c1 - 1);
+#pragma unroll
+      for (int n = 0; n < NC; ++n) kb[u][n] = *gptr<u32x4>(kp + row * D + (4 * n + lq) * EPC);
     }
-    if (valid && sub == 0) p.acc[off + j] += sc;
+  };
+  u32x4 qb[NC];
+  {
+    const T* qs = (const T*)p.q + ((int64_t)s * nh + min(lc, nh - 1)) * D;
+    const bool al = ((uintptr_t)p.q & 15) == 0;
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+      qb[n] = load_chunk<T>(qs + (4 * n + lq) * EPC, al);
+      if (lc >= nh) qb[n] = u32x4{0, 0, 0, 0};
+    }
+  }
+  if (w < ntiles) load(w);
+  float m = kNegBigS, l = 0.f;  // SCORE 0: running statistics of head lc; SCORE 1: its (max, 1 / sum)
+  if constexpr (SCORE) {
+    // merge the slices' statistics: wave w takes heads w, w + NW, ...
+    for (int h = w; h < nh; h += NW) {
+      const WNW_GLOBAL float* pp = gptr<float>(p.part) + ((int64_t)s * C * nh + h) * 2;
+      float mq[2], lsum[2];  // C <= 128
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int i = lane + 64 * k;
+        mq[k] = i < C ? pp[(int64_t)min(i, C - 1) * nh * 2] : kNegBigS;
+        lsum[k] = i < C ? pp[(int64_t)min(i, C - 1) * nh * 2 + 1] : 0.f;
+      }
+      const float M = wave_max(fmaxf(mq[0], mq[1]));
+      const float L = wave_sum(lsum[0] * exp2f(mq[0] - M) + lsum[1] * exp2f(mq[1] - M));
+      if (lane == 0) {
+        stat[h][0] = M;
+        stat[h][1] = 1.f / L;
+      }
+    }
+    __syncthreads();
+    m = stat[min(lc, nh - 1)][0];
+    l = lc < nh ? stat[lc][1] : 0.f;
+  }
+  for (int t0 = w; t0 < ntiles; t0 += NW * U) {
+    f32x4 x[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      x[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int n = 0; n < NC; ++n) x[u] = dot_chunk<T>(kb[u][n], qb[n], x[u]);
+    }
+    if (t0 + NW * U < ntiles) load(t0 + NW * U);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t row = c0 + 16 * (int64_t)(t0 + NW * u) + 4 * lq;  // of x[u][0]
+      if constexpr (SCORE) {
+        float sc[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          sc[i] = lc < nh ? exp2f(x[u][i] * p.scale_log2 - m) * l : 0.f;
+          // the 16 heads of the lane's row group
+#pragma unroll
+          for (int o = 8; o >= 1; o >>= 1) sc[i] += __shfl_xor(sc[i], o);
+        }
+        const float mine = lc == 0 ? sc[0] : lc == 1 ? sc[1] : lc == 2 ? sc[2] : sc[3];
+        if (lc < 4 && row + lc < c1) {
+          WNW_GLOBAL float* a = gptr_w<float>(p.acc) + off + (row + lc - a_row);
+          *a += mine;
+        }
+      } else {
+        float v[4], mx = m;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          v[i] = row + i < c1 ? x[u][i] * p.scale_log2 : -INFINITY;
+          mx = fmaxf(mx, v[i]);
+        }
+        l *= exp2f(m - mx);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) l += exp2f(v[i] - mx);
+        m = mx;
+      }
+    }
+  }
+  if constexpr (!SCORE) {
+#pragma unroll
+    for (int o = 16; o < 64; o <<= 1) {  // the lane quarters of head lc
+      const float m2 = __shfl_xor(m, o), l2 = __shfl_xor(l, o);
+      merge_ml(m, l, m2, l2);
+    }
+    if (lane < 16) {
+      red[w][lane][0] = m;
+      red[w][lane][1] = l;
+    }
+    __syncthreads();
+    if (tid < nh) {
+      float M = kNegBigS, L = 0.f;
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) merge_ml(M, L, red[ww][tid][0], red[ww][tid][1]);
+      WNW_GLOBAL float* out = gptr_w<float>(p.part) + (((int64_t)s * C + c) * nh + tid) * 2;
+      out[0] = M;
+      out[1] = L;
+    }
   }
 }
 
-enum ScoreKernel { kAttnScore = 0, kSegStats = 1, kSegScore = 2 };
-
-template <typename T, int D>
-static const void* score_fn(int which, int iters) {
-  const bool small = iters == kItersSmall;
-  switch (which) {
-    case kAttnScore:
-      return small ? (const void*)&attn_score_kernel<T, D, kItersSmall> : (const void*)&attn_score_kernel<T, D, kIters>;
-    case kSegStats: return (const void*)&seg_stats_kernel<T, D>;
-    case kSegScore:
-      return small ? (const void*)&seg_score_kernel<T, D, kItersSmall> : (const void*)&seg_score_kernel<T, D, kIters>;
-  }
-  return nullptr;
-}
-
-template <typename T>
-static const void* score_fn_d(int which, int64_t D, int iters) {
+// Calls f with a T and the head_dim as compile-time constants; false for a
+// type or head_dim without an instance.
+template <typename F, typename T>
+static bool with_dim(int64_t D, F f, T t) {
   switch (D) {
-    case 64: return score_fn<T, 64>(which, iters);
-    case 128: return score_fn<T, 128>(which, iters);
-    case 256: return score_fn<T, 256>(which, iters);
+    case 64: return f(t, std::integral_constant<int, 64>()), true;
+    case 128: return f(t, std::integral_constant<int, 128>()), true;
+    case 256: return f(t, std::integral_constant<int, 256>()), true;
   }
-  return nullptr;
+  return false;
+}
+template <typename F>
+static bool with_type(int dtype, int64_t D, F f) {
+  switch (dtype) {
+    case WNW_BF16: return with_dim(D, f, bf16_t());
+    case WNW_F16: return with_dim(D, f, f16_t());
+    case WNW_F32: return with_dim(D, f, float());
+  }
+  return false;
 }
 
 // Rows per iteration count for a scoring grid of `ny` rows of workgroups over
@@ -469,19 +542,6 @@ static int score_iters(int64_t max_audio, int64_t ny, int64_t head_dim, int elem
   const int cus = device_cus();
   const int64_t rows16 = score_rows_per_wg((int)head_dim, elem_bytes, kIters);
   return ((max_audio + rows16 - 1) / rows16) * ny >= 2 * (int64_t)cus ? kIters : kItersSmall;
-}
-
-template <typename P>
-static hipError_t launch_score(int which, int dtype, int64_t D, int iters, dim3 grid, P prm, hipStream_t st) {
-  const void* fn = nullptr;
-  switch (dtype) {
-    case WNW_BF16: fn = score_fn_d<bf16_t>(which, D, iters); break;
-    case WNW_F16: fn = score_fn_d<f16_t>(which, D, iters); break;
-    case WNW_F32: fn = score_fn_d<float>(which, D, iters); break;
-  }
-  if (!fn) return hipErrorInvalidValue;
-  void* args[] = {&prm};
-  return hipLaunchKernel(fn, grid, dim3(kScoreThreads), args, 0, st);
 }
 
 }  // namespace wnw
@@ -579,8 +639,13 @@ static int decode_attn_score_impl(const void* q, const void* k, const void* v, c
   const int iters = score_iters(max_audio, n_seg / num_kv_heads, head_dim, elem_bytes(dtype));
   const int rows_wg = score_rows_per_wg((int)head_dim, elem_bytes(dtype), iters);
   const dim3 grid((unsigned)((max_audio + rows_wg - 1) / rows_wg), (unsigned)(n_seg / num_kv_heads));
-  WNW_CHECK_HIP(launch_score(kAttnScore, dtype, head_dim, iters, grid, sp, (hipStream_t)stream),
-                "attention score launch");
+  const bool known = with_type(dtype, head_dim, [&](auto t, auto d) {
+    typedef decltype(t) T;
+    constexpr int D = decltype(d)::value;
+    hipLaunchKernelGGL((iters == kIters ? attn_score_kernel<T, D, kIters> : attn_score_kernel<T, D, kItersSmall>), grid,
+                       dim3(kScoreThreads), 0, (hipStream_t)stream, sp);
+  });
+  WNW_CHECK_HIP(known ? hipGetLastError() : hipErrorInvalidValue, "attention score launch");
   return WNW_OK;
 }
 
@@ -725,7 +790,7 @@ extern "C" int wnw_decode_attn_append_deferred(
 
 extern "C" int64_t wnw_fused_score_workspace_bytes(int64_t n_samples, int64_t n_heads) {
   if (n_samples < 0 || n_heads <= 0) return -1;
-  return up256(n_samples * kStatChunks * n_heads * 2 * 4);
+  return up256(n_samples * score_slices(n_samples) * n_heads * 2 * 4);
 }
 
 extern "C" int wnw_fused_score_accumulate(const void* q, const void* k, const int32_t* seg_starts,
@@ -763,12 +828,14 @@ extern "C" int wnw_fused_score_accumulate(const void* q, const void* k, const in
   sp.nh = (int32_t)n_heads;
   sp.scale_log2 = scale * kLog2eS;
   hipStream_t st = (hipStream_t)stream;
-  WNW_CHECK_HIP(launch_score(kSegStats, dtype, head_dim, kIters, dim3(kStatChunks, (unsigned)n_samples), sp, st),
-                "score statistics launch");
-  const int iters = score_iters(max_audio, n_samples, head_dim, elem_bytes(dtype));
-  const int rows_wg = score_rows_per_wg((int)head_dim, elem_bytes(dtype), iters);
-  const dim3 grid((unsigned)((max_audio + rows_wg - 1) / rows_wg), (unsigned)n_samples);
-  WNW_CHECK_HIP(launch_score(kSegScore, dtype, head_dim, iters, grid, sp, st), "score launch");
+  const dim3 grid((unsigned)score_slices(n_samples), (unsigned)n_samples);
+  const bool known = with_type(dtype, head_dim, [&](auto t, auto d) {
+    typedef decltype(t) T;
+    constexpr int D = decltype(d)::value;
+    hipLaunchKernelGGL((seg_score_kernel<T, D, false>), grid, dim3(kScoreThreads), 0, st, sp);
+    hipLaunchKernelGGL((seg_score_kernel<T, D, true>), grid, dim3(kScoreThreads), 0, st, sp);
+  });
+  WNW_CHECK_HIP(known ? hipGetLastError() : hipErrorInvalidValue, "score launch");
   return WNW_OK;
 }
 
