@@ -671,6 +671,56 @@ int wnw_gather_host_rows(const void* host_k, const void* host_v,
                          int64_t out_rows, void* stream);
 
 /* ------------------------------------------------------------------------ */
+/* Prompt (the session's prefill branch)                                     */
+/* ------------------------------------------------------------------------ */
+
+/*
+ * Causal attention of a whole prompt, the scaled_dot_product_attention call
+ * of src/algorithms/wnw/code/session.py:56-59 without a mask:
+ *   out[b, h, i] = softmax_j<=i(scale * q[b, h, i] . k[b, h', j]) @ v[b, h']
+ * with h' = h / (n_heads / n_kv_heads).  strides: 12 element strides (batch,
+ * head, row) of q, k, v and out, multiples of 16 bytes; head_dim is
+ * contiguous.  bf16 / f16, head_dim 64 or 128, scale > 0 (WNW_ENOTSUP
+ * otherwise).  32-bit scores, softmax and sums; the weights enter the value
+ * product in the inputs' type.
+ */
+int wnw_prefill_attn(const void* q, const void* k, const void* v, int64_t batch,
+                     int64_t n_heads, int64_t n_kv_heads, int64_t seq,
+                     int64_t head_dim, const int64_t* strides, float scale,
+                     int dtype, void* out, void* stream);
+
+/*
+ * Prompt token scores of one layer (src/algorithms/wnw/code/session.py:
+ * 119-170), two launches.  q [batch, heads, seq, head_dim], k [batch,
+ * kv_heads, seq, head_dim]; strides: element strides (batch, head, row) of q
+ * and k (multiples of 16 bytes, head_dim contiguous), then (batch, row) of
+ * mask, an additive [batch, 1, seq, seq] of mask_dtype with contiguous rows,
+ * or null: causal.  With w the softmax over all keys of scale * q . k + mask
+ * and [audio_starts[b], audio_ends[b]) each sample's audio rows (host arrays):
+ *   out_a[b, j] = sum over the n_a heads a_heads (against KV head a_heads[0] /
+ *       group) of the last row's w at audio row j;
+ *   out_h[b, i, j] = sum over the heads of KV head kv_heads[i] of w at audio
+ *       row j, of the last row (last_row != 0) or averaged over the rows after
+ *       the audio (0 where there are none).
+ * max_audio: row length of out_a / out_h; max_queries >= group x rows of any
+ * sample and n_a.  head_dim 64, 128 or 256, at most 64 samples, class-A heads
+ * and KV heads (WNW_ENOTSUP otherwise).
+ */
+int64_t wnw_prefill_scores_workspace_bytes(int64_t batch, int64_t n_items,
+                                           int64_t seq, int64_t head_dim,
+                                           int64_t max_queries, int dtype);
+int wnw_prefill_scores(const void* q, const void* k, const void* mask,
+                       const int64_t* strides, int64_t batch, int64_t group,
+                       int64_t seq, int64_t head_dim,
+                       const int32_t* audio_starts, const int32_t* audio_ends,
+                       const int32_t* a_heads, int64_t n_a,
+                       const int32_t* kv_heads, int64_t n_kv, int last_row,
+                       float scale, int dtype, int mask_dtype,
+                       int64_t max_audio, int64_t max_queries, float* out_a,
+                       float* out_h, void* workspace, int64_t workspace_bytes,
+                       void* stream);
+
+/* ------------------------------------------------------------------------ */
 /* Measurement                                                               */
 /* ------------------------------------------------------------------------ */
 

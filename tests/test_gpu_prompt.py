@@ -1,0 +1,145 @@
+"""The prompt kernels against 64-bit attention, and the inputs they leave to
+PyTorch.
+
+Attention: 16-bit outputs and 16-bit weights in the value product, relative
+2-norm error of at most 4e-3 (bf16, 2^-8 steps) / 5e-4 (f16).  Scores: 32-bit
+logits of exact 16-bit products, 32-bit sums: 1e-6 + 1e-4 |ref| (weights in
+[0, 1], the exponential's argument error scales with the logits)."""
+import pytest
+import torch
+
+from wnw_amd import _lib
+from wnw_amd.wnw import prompt, session
+
+pytestmark = pytest.mark.gpu
+
+
+def _qkv(dev, B, H, S, D, dtype, seed, layout):
+    g = torch.Generator(device=dev)
+    g.manual_seed(seed)
+    if layout == "rows":  # [B, S, H, D] viewed as [B, H, S, D], as projections leave it
+        return [torch.randn(B, S, H, D, device=dev, generator=g).to(dtype).transpose(1, 2) for _ in range(3)]
+    return [torch.randn(B, H, S, D, device=dev, generator=g).to(dtype) for _ in range(3)]
+
+
+@pytest.mark.parametrize("S", [1, 2, 31, 32, 33, 63, 64, 65, 127, 128, 129, 193, 500])
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.float16, 128), (torch.bfloat16, 64)])
+@pytest.mark.parametrize("layout", ["heads", "rows"])
+def test_causal_attention(gpu, S, dtype, D, layout):
+    q, k, v = _qkv(gpu, 2, 3, S, D, dtype, S, layout)
+    out = session.prefill_attention(q, k, v, None, 0.11)
+    assert prompt.causal_attention(q, k, v, 0.11) is not None
+    assert out.stride() == q.stride() and out.dtype == dtype
+    s = (q.double() @ k.double().transpose(-1, -2).contiguous()) * 0.11
+    s = s + torch.full((S, S), float("-inf"), device=gpu, dtype=torch.float64).triu_(1)
+    ref = s.softmax(-1) @ v.double().contiguous()
+    err = float((out.double() - ref).norm() / ref.norm())
+    assert err < (4e-3 if dtype == torch.bfloat16 else 5e-4), err
+
+
+def test_causal_attention_large_scores(gpu):
+    """Scores in the thousands and equal rows: the running maximum carries the
+    sums, no overflow."""
+    q, k, v = _qkv(gpu, 1, 2, 300, 128, torch.bfloat16, 9, "heads")
+    q = q * 30
+    k[:, :, 100:140] = k[:, :, 100:101]
+    ref = ((q.double() @ k.double().transpose(-1, -2).contiguous()) +
+           torch.full((300, 300), float("-inf"), device=gpu, dtype=torch.float64).triu_(1)).softmax(-1) @ v.double()
+    out = prompt.causal_attention(q, k, v, 1.0)
+    assert float((out.double() - ref).norm() / ref.norm()) < 4e-3
+
+
+def test_inputs_left_to_torch(gpu):
+    q, k, v = _qkv(gpu, 1, 2, 40, 128, torch.bfloat16, 3, "heads")
+    assert prompt.causal_attention(q, k, v, 0.1) is not None
+    assert prompt.causal_attention(q, k, v, -0.1) is None  # the running maximum needs a positive scale
+    assert prompt.causal_attention(q, k[:, :, :30], v[:, :, :30], 0.1) is None
+    assert prompt.causal_attention(q.float(), k.float(), v.float(), 0.1) is None
+    wide = torch.randn(1, 2, 40, 129, device=gpu).to(torch.bfloat16)
+    assert prompt.causal_attention(wide[..., 1:], k, v, 0.1) is None  # rows not 16-byte aligned
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    assert prompt.causal_attention(q, k, v, 0.1) is None
+    out = session.prefill_attention(q, k, v, None, 0.1)
+    out.float().sum().backward()
+    assert q.grad is not None and k.grad is not None and v.grad is not None
+    with torch.no_grad():
+        assert prompt.causal_attention(q, k, v, 0.1) is not None
+    q, k, v = (t.detach() for t in (q, k, v))
+    got = torch.func.vmap(lambda a: session.prefill_attention(a, k, v, None, 0.1))(torch.stack([q, q]))
+    torch.testing.assert_close(got[0], session.prefill_attention(q, k, v, None, 0.1), atol=2e-2, rtol=2e-2)
+
+
+class _Config:
+    def __init__(self, a_heads, group, mode):
+        self.prefill_score_mode, self._a, self._g = mode, a_heads, group
+
+    def get_layer_class_a(self, layer):
+        return self._a
+
+    def is_class_a_kv_head(self, layer, h):
+        return h in {x // self._g for x in self._a}
+
+
+class _Cache:
+    def __init__(self, config, starts, ends):
+        self.config, self._raw_audio_starts, self._raw_audio_ends = config, starts, ends
+
+
+@pytest.mark.parametrize("dtype,D,G,H,S", [(torch.bfloat16, 128, 4, 4, 700), (torch.float16, 64, 7, 2, 257),
+                                           (torch.float32, 128, 2, 3, 300), (torch.bfloat16, 256, 1, 2, 65),
+                                           (torch.float32, 256, 3, 2, 130)])
+@pytest.mark.parametrize("mode", ["last", "mean_text"])
+@pytest.mark.parametrize("mask", ["none", "float", "bool", "lowest"])
+def test_token_scores(gpu, dtype, D, G, H, S, mode, mask):
+    """Two samples: text after the audio of one (more queries than fit the LDS
+    at a time at 700 rows), none after the other's; masks additive, boolean,
+    and with the type's lowest value instead of -inf."""
+    B, starts, ends = 2, [5, 1], [S // 3, S]
+    q = _qkv(gpu, B, G * H, S, D, dtype, 1, "rows")[0]
+    k = _qkv(gpu, B, H, S, D, dtype, 2, "heads")[0]
+    base = torch.ones(B, 1, S, S, device=gpu).tril_().bool()
+    base[1, :, :, :2] = False
+    base[1, :, :2, :2] = True
+    m = {"none": None, "bool": base,
+         "float": torch.where(base, 0.0, float("-inf")).to(dtype) + torch.rand(S, device=gpu).to(dtype),
+         "lowest": torch.where(base, 0.0, torch.finfo(dtype).min).to(dtype)}[mask]
+    a_heads = [0, G - 1] if G > 1 else [0]
+    cache = _Cache(_Config(a_heads, G, mode), starts, ends)
+    got = session.compute_prefill_scores(q, k, m, cache, 0, H, G, D ** -0.5)
+    m64 = None if m is None else (torch.where(m, 0.0, float("-inf")) if mask == "bool" else m).double()
+    want = _scores64(q.double(), k.double(), m64, cache, H, G, D ** -0.5)
+    assert _lib.device_error() == 0
+    for b in range(B):
+        pairs = [(got[0][b], want[0][b])] + list(zip(got[1][b], want[1][b]))
+        for x, y in pairs:
+            assert (x is None) == (y is None)
+            if x is not None:
+                assert x.dtype == torch.float32 and x.shape == y.shape
+                torch.testing.assert_close(x.double(), y, atol=1e-6, rtol=1e-4)
+
+
+def _scores64(q, k, m, cache, H, G, scale):
+    """compute_prefill_scores in 64 bits."""
+    B, _, S, _ = q.shape
+    if m is None:
+        m = torch.full((S, S), float("-inf"), device=q.device, dtype=torch.float64).triu_(1).expand(B, 1, S, S)
+    cfg = cache.config
+    a, per = [], []
+    for b in range(B):
+        ra, re = cache._raw_audio_starts[b], cache._raw_audio_ends[b]
+        ca = cfg.get_layer_class_a(0)
+        a.append(((q[b, ca, -1] @ k[b, ca[0] // G].t()) * scale + m[b, 0, -1]).softmax(-1)[:, ra:re].sum(0))
+        row = []
+        for h in range(H):
+            if cfg.is_class_a_kv_head(0, h):
+                row.append(None)
+                continue
+            rows = slice(S - 1, S) if cfg.prefill_score_mode == "last" else slice(re, S)
+            if rows.start == S:
+                row.append(torch.zeros(re - ra, device=q.device, dtype=torch.float64))
+                continue
+            s = (q[b, h * G:(h + 1) * G, rows] @ k[b, h].t()) * scale + m[b, 0, rows]
+            row.append(s.softmax(-1)[:, :, ra:re].mean(dim=1).sum(0))
+        per.append(row)
+    return a, per

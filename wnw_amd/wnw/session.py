@@ -28,6 +28,7 @@ from torch import Tensor
 
 from ..kv.flat_cache import FlatVarlenCache
 from ..kv.fused_attn import q1_decode_attn
+from .prompt import causal_attention, token_scores
 
 
 def fused_attn_enabled() -> bool:
@@ -74,10 +75,17 @@ def prefill_attention(q: Tensor, k: Tensor, v: Tensor, attention_mask: Tensor | 
     the model's mask, causal when there is none).  q/k/v: [B, Hq, S, D]
     (K/V already repeated over the group).
 
-    SDPA runs with its fused backends only (flash, memory-efficient); when
-    neither takes the inputs, the same attention is computed in float32
-    over query chunks with contiguous operands (the products in float32,
-    so no batched bf16 product with a transposed operand is issued)."""
+    Without a mask, GPU inputs in 16 bits run the prompt kernel (head_dim
+    64 or 128, nothing to differentiate; 4,564 rows of 32 heads at head_dim
+    128: 211 us against SDPA's 588).  Otherwise SDPA runs with its fused
+    backends only (flash, memory-efficient); when neither takes the inputs,
+    the same attention is computed in float32 over query chunks with
+    contiguous operands (the products in float32, so no batched bf16 product
+    with a transposed operand is issued)."""
+    if attention_mask is None:
+        out = causal_attention(q, k, v, scaling)
+        if out is not None:
+            return out
     from torch.nn.attention import SDPBackend, sdpa_kernel
 
     try:
@@ -110,10 +118,19 @@ def compute_prefill_scores(q: Tensor, k: Tensor, attention_mask: Tensor | None, 
     """Prefill token scores (session.py:119-169): class-A scores from the
     last prompt token of the layer's class-A query heads against their KV
     head, and per class-B/other KV head scores by ``prefill_score_mode``
-    ("last": last token; "mean_text": mean over the text after the audio)."""
+    ("last": last token; "mean_text": mean over the text after the audio).
+    On the GPU two launches per layer; the PyTorch form below them serves the
+    other inputs (CPU, other shapes, autograd)."""
     B, _, S, _ = q.shape
     if attention_mask is not None and attention_mask.dim() == 4 and attention_mask.dtype == torch.bool:
         attention_mask = torch.where(attention_mask, 0.0, float("-inf")).to(q.dtype)
+    others = [h for h in range(num_kv_heads) if not cache.config.is_class_a_kv_head(layer_idx, h)]
+    scores = token_scores(q, k, attention_mask, cache._raw_audio_starts, cache._raw_audio_ends,
+                          cache.config.get_layer_class_a(layer_idx), others, num_kv_groups,
+                          cache.config.prefill_score_mode == "last", scaling)
+    if scores is not None:
+        place = {h: i for i, h in enumerate(others)}
+        return scores[0], [[row[place[h]] if h in place else None for h in range(num_kv_heads)] for row in scores[1]]
     if attention_mask is None:
         causal = torch.full((S, S), float("-inf"), device=q.device, dtype=q.dtype).triu_(1)
         attention_mask = causal.unsqueeze(0).unsqueeze(0).expand(B, 1, S, S)
