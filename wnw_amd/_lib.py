@@ -120,6 +120,25 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_callpath = None
+
+
+def callpath():
+    """The native form of the operators' plain calls (``_callpath.so``, built
+    with the library; raises if it has not been)."""
+    global _callpath
+    if _callpath is None:
+        lib()
+        from . import _callpath as mod
+        from .kv.fused_attn import call_workspace
+        from .wnw.kernels import call_score_workspace
+
+        mod.setup(_raw_stream if _raw_stream is not None else lambda i: raw_stream(torch.device("cuda", i)),
+                  call_workspace, call_score_workspace, check)
+        _callpath = mod
+    return _callpath
+
+
 class WnwError(RuntimeError):
     pass
 
@@ -177,7 +196,10 @@ _init_done: set[int] = set()
 
 
 def ensure_init(device: torch.device) -> None:
-    idx = device.index if device.index is not None else torch.cuda.current_device()
+    ensure_init_index(device.index if device.index is not None else torch.cuda.current_device())
+
+
+def ensure_init_index(idx: int) -> None:
     if idx in _init_done:
         return
     with torch.cuda.device(idx):

@@ -72,6 +72,22 @@ def rebuild_append_kv(
 
 
 _score_ws: dict[tuple[int, int], torch.Tensor] = {}
+_score_need: dict[tuple[int, int], int] = {}  # bytes the library asks for, per (items, heads)
+
+
+def call_score_workspace(idx: int, stream: int, items: int, heads: int) -> torch.Tensor:
+    """The scoring workspace of a call on ``stream`` of device ``idx``."""
+    _lib.ensure_init_index(idx)
+    need = _score_need.get((items, heads))
+    if need is None:
+        need = int(_lib.lib().wnw_fused_score_workspace_bytes(items, heads))
+        if len(_score_need) < 4096:
+            _score_need[(items, heads)] = need
+    ws = _score_ws.get((idx, stream))
+    if ws is None or ws.numel() < need:
+        ws = torch.empty(max(need, 1 << 16), dtype=torch.uint8, device=torch.device("cuda", idx))
+        _score_ws[(idx, stream)] = ws
+    return ws
 
 
 def fused_score_accumulate(
@@ -98,6 +114,11 @@ def fused_score_accumulate(
     defaults to d^-0.5 like the reference; ``max_audio`` (largest audio
     range) is read back from the device when not given.
     """
+    if max_audio is not None:  # the plain form: checked and launched natively, 18 -> 6.1 us of host time
+        if (_lib._callpath or _lib.callpath()).score(
+                Q, K, seg_starts, seg_ends, audio_starts, audio_ends, accumulator, accum_offsets, max_audio,
+                Q.shape[-1] ** -0.5 if scale is None else scale):
+            return
     _lib.require_gpu(Q, K, seg_starts, seg_ends, audio_starts, audio_ends, accumulator, accum_offsets)
     S, nh, d = Q.shape
     for name, t, n in (("seg_starts", seg_starts, S), ("seg_ends", seg_ends, S), ("audio_starts", audio_starts, S),
@@ -122,15 +143,9 @@ def fused_score_accumulate(
     Q = Q.contiguous()
     seg_starts, seg_ends, audio_starts, audio_ends, accum_offsets = (
         t.contiguous() for t in (seg_starts, seg_ends, audio_starts, audio_ends, accum_offsets))
-    need = int(_lib.lib().wnw_fused_score_workspace_bytes(S, nh))
     dev = Q.device
-    key = (dev.index if dev.index is not None else torch.cuda.current_device(),
-           torch.cuda.current_stream(dev).cuda_stream)
-    ws = _score_ws.get(key)
-    if ws is None or ws.numel() < need:
-        ws = torch.empty(max(need, 1 << 16), dtype=torch.uint8, device=dev)
-        _score_ws[key] = ws
-    _lib.ensure_init(dev)
+    ws = call_score_workspace(dev.index if dev.index is not None else torch.cuda.current_device(),
+                              _lib.raw_stream(dev), S, nh)
     _lib.check(_lib.lib().wnw_fused_score_accumulate(
         _lib.ptr(Q), _lib.ptr(K), _lib.ptr(seg_starts), _lib.ptr(seg_ends), _lib.ptr(audio_starts),
         _lib.ptr(audio_ends), _lib.ptr(accumulator), _lib.ptr(accum_offsets), S, nh, d, K.shape[0],
