@@ -49,6 +49,23 @@ def test_causal_attention_large_scores(gpu):
     assert float((out.double() - ref).norm() / ref.norm()) < 4e-3
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 4e-3), (torch.float16, 5e-4)])
+@pytest.mark.parametrize("step", [2.0, 7.5, 8.5])
+def test_causal_attention_rising_scores(gpu, dtype, tol, step):
+    """The weights' reference trails the maximum by up to 8 (log2): scores
+    that rise by less and by more than that from one 64-key tile to the next,
+    and fall again.  A weight's relative rounding does not depend on the
+    reference, so the bounds are the ones above."""
+    q, k, v = _qkv(gpu, 1, 2, 700, 128, dtype, 11, "heads")
+    q[..., 0] = 8.0
+    tiles = torch.tensor([0, 1, 2, 3, 3, 4, 2, 5, 0, 6, 7], device=gpu, dtype=torch.float32)
+    k[..., 0] = (tiles.repeat_interleave(64)[:700] * (step * 0.6931 / (8.0 * 0.08))).to(dtype)
+    ref = ((q.double() @ k.double().transpose(-1, -2).contiguous()) * 0.08 +
+           torch.full((700, 700), float("-inf"), device=gpu, dtype=torch.float64).triu_(1)).softmax(-1) @ v.double()
+    out = prompt.causal_attention(q, k, v, 0.08)
+    assert float((out.double() - ref).norm() / ref.norm()) < tol
+
+
 def test_inputs_left_to_torch(gpu):
     q, k, v = _qkv(gpu, 1, 2, 40, 128, torch.bfloat16, 3, "heads")
     assert prompt.causal_attention(q, k, v, 0.1) is not None

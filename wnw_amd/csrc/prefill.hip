@@ -81,13 +81,23 @@ struct PromptOps<float> {
 //       keys 8 j + 4 hi + 0..3 of query n, which is already the P^T operand
 //       when V^T's k-slots follow the same order: two ds_read_b64_tr_b16 per
 //       operand (4 keys x 1 column per lane each; V chunks swizzled by 2 (row % 4)).
-// Online softmax in-lane (queries are columns); the sums are rescaled only in
-// tiles where some query's maximum grew.  P goes through 16 bits, its sum
-// stays 32-bit.  Bound by the matrix cores, the LDS reads of their operands
-// and the exponentials about evenly; two workgroups per CU let one wave's
-// softmax run beside another's products.  bf16, D = 128, 32 heads: 4,564 rows
-// 588 us (SDPA's flash kernel, 290 TFLOP/s) -> 211 us (810), 7,564 rows 1,306 ->
-// 550 us; the same error against 64 bits.
+// Online softmax in-lane (queries are columns), against a reference that trails
+// the running maximum by up to 2^kPaLag: the sums are rescaled only in tiles
+// where some query's maximum passed that (with 32 queries per wave one of them
+// grows in most of the first 50 tiles; 66 of 207 vector instructions a tile).
+// The weights are then up to 2^8 instead of 1, which their rounding to 16 bits
+// (relative) and the 32-bit sums do not see.  Only the diagonal tile masks, and
+// only the last tile clamps its rows.  P goes through 16 bits, its sum stays
+// 32-bit.
+// Bound by the issue of vector instructions (exponentials above all) beside
+// the matrix instructions: two waves per SIMD overlap them only in part.
+// bf16, D = 128, 32 heads: 4,564 rows 588 us (SDPA's flash kernel, 290 TFLOP/s) ->
+// 183 us (933; 202 with every growth rescaled, a mask in every tile and the
+// copies' offsets worked out per tile), 2 x 28 heads of 2,000 rows 85 -> 71 us; the
+// same error against 64 bits.  Measured and not kept: 64 queries per wave and
+// one wave per SIMD (306 us: sums move through accumulator registers), the next
+// tile's scores issued ahead of a tile's softmax (189-190 against 194 us, more
+// registers), the first values of a tile read ahead of its softmax (the same).
 struct PromptAttnParams {
   const void *q, *k, *v;
   void* out;
@@ -98,6 +108,7 @@ struct PromptAttnParams {
 
 static constexpr int kPaQ = 128;   // queries per workgroup
 static constexpr int kPaKeys = 64;  // keys per tile
+static constexpr float kPaLag = 8.f;  // log2 of the largest weight before the sums are rescaled
 
 // 16 bytes per lane from gbase + voff into LDS at lds_addr + 16 * lane (M0
 // carries the LDS address and is restored).
@@ -144,18 +155,29 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PromptAttnParams p
   }
   const uint32_t lds0 =
       __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)lds);
-  auto issue = [&](int tile, int buf) {
-    const int key0 = tile * kPaKeys;
-    const void* kt = uniform_ptr(kp + (int64_t)key0 * p.ks);
-    const void* vt = uniform_ptr(vp + (int64_t)key0 * p.vs);
-    const uint32_t dst = lds0 + buf * 2 * TB;
-    const int last = S - 1 - key0;  // rows past the prompt repeat its last (masked: later than every query)
+  // lane offsets of a tile's copies: those of a whole tile, until the last one clamps its rows
+  uint32_t kdma[NI], vdma[NI];
+  auto copy_offsets = [&](int last) {
 #pragma unroll
     for (int u = 0; u < NI; ++u) {
       const int r = (w * NI + u) * RPI + lane / CH;
       const int rr = min(r, last), c = lane % CH;
-      prompt_copy16(kt, (uint32_t)(rr * (int)p.ks * 2 + (c ^ (r % CH)) * 16), dst + (w * NI + u) * 1024);
-      prompt_copy16(vt, (uint32_t)(rr * (int)p.vs * 2 + (c ^ (2 * (r & 3))) * 16), dst + TB + (w * NI + u) * 1024);
+      kdma[u] = (uint32_t)(rr * (int)p.ks * 2 + (c ^ (r % CH)) * 16);
+      vdma[u] = (uint32_t)(rr * (int)p.vs * 2 + (c ^ (2 * (r & 3))) * 16);
+    }
+  };
+  copy_offsets(kPaKeys - 1);
+  auto issue = [&](int tile, int buf) {  // tiles in ascending order
+    const int key0 = tile * kPaKeys;
+    const void* kt = uniform_ptr(kp + (int64_t)key0 * p.ks);
+    const void* vt = uniform_ptr(vp + (int64_t)key0 * p.vs);
+    const uint32_t dst = lds0 + buf * 2 * TB;
+    // rows past the prompt repeat its last (masked: later than every query)
+    if (key0 + kPaKeys > S) copy_offsets(S - 1 - key0);
+#pragma unroll
+    for (int u = 0; u < NI; ++u) {
+      prompt_copy16(kt, kdma[u], dst + (w * NI + u) * 1024);
+      prompt_copy16(vt, vdma[u], dst + TB + (w * NI + u) * 1024);
     }
   };
   // lane offsets of the operands inside a tile
@@ -172,26 +194,21 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PromptAttnParams p
   f32x16 o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) o[dt] = f32x16{};
-  float m = -3.402823466e38f, l = 0.f;  // below every score (a fully masked value is -inf)
+  // the reference of the weights: below every score (a fully masked value is -inf)
+  float m = -3.402823466e38f, l = 0.f;
   const int ntile = min((qblk + 1) * (kPaQ / kPaKeys), (S + kPaKeys - 1) / kPaKeys);
-  const int mine = (q0 + 31) / kPaKeys;  // the wave's diagonal tile
-  issue(0, 0);
-  for (int i = 0; i < ntile; ++i) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();  // tile i has landed; everyone is done with tile i - 1
-    if (i + 1 < ntile) issue(i + 1, (i + 1) & 1);
-    if (i > mine) continue;
+  const int mine = min((q0 + 31) / kPaKeys, ntile - 1);  // the wave's diagonal tile
+  auto tile = [&](int i, auto masked) {
     const uint8_t* kt = lds[i & 1];
     const uint8_t* vt = kt + TB;
     f32x16 s[2];
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      s[mt] = f32x16{};
+    for (int mt = 0; mt < 2; ++mt) s[mt] = f32x16{};
 #pragma unroll
-      for (int kk = 0; kk < KK; ++kk)
-        s[mt] = Ops::mma32(*(const u32x4*)(kt + koff[kk] + mt * 32 * RB), qr[kk], s[mt]);
-    }
-    if (i == mine || (i + 1) * kPaKeys > S) {
+    for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt) s[mt] = Ops::mma32(*(const u32x4*)(kt + koff[kk] + mt * 32 * RB), qr[kk], s[mt]);
+    if constexpr (decltype(masked)::value) {
       const int lim = qi - i * kPaKeys - 4 * hi;  // keys 32 mt + 8 j + c (+ 4 hi) up to the query
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt)
@@ -205,7 +222,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PromptAttnParams p
 #pragma unroll
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[mt][r]);
     mx = max_x32(mx);
-    if (__ballot(mx > m)) {
+    if (__ballot((mx - m) * p.scale_log2 > kPaLag)) {
       const float alpha = __builtin_amdgcn_exp2f((m - mx) * p.scale_log2);
       l *= alpha;
 #pragma unroll
@@ -224,6 +241,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PromptAttnParams p
         pb[kk][j] = Ops::pack2(x0, x1);
       }
     }
+    __builtin_amdgcn_s_setprio(1);  // a wave at its products before another's softmax: 185 -> 183 us
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
@@ -233,7 +251,23 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PromptAttnParams p
         const u32x4 a = u32x4{(uint32_t)v0, (uint32_t)(v0 >> 32), (uint32_t)v1, (uint32_t)(v1 >> 32)};
         o[dt] = Ops::mma32(a, pb[kk], o[dt]);
       }
+    __builtin_amdgcn_s_setprio(0);
+  };
+  auto turn = [&](int i) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();  // tile i has landed; everyone is done with tile i - 1
+    if (i + 1 < ntile) issue(i + 1, (i + 1) & 1);
+  };
+  issue(0, 0);
+  // the tiles up to the wave's diagonal, the diagonal one, the turns of the
+  // workgroup's later waves
+  for (int i = 0; i < mine; ++i) {
+    turn(i);
+    tile(i, std::false_type());
   }
+  turn(mine);
+  tile(mine, std::true_type());
+  for (int i = mine + 1; i < ntile; ++i) turn(i);
   if (qi >= S) return;
   const float inv = 1.f / sum_x32(l);
   T* op = (T*)p.out + b * p.ob + h * p.oh + (int64_t)qi * p.os;
