@@ -71,6 +71,8 @@ def test_refusals_and_transforms(gpu):
             decode_attn(q, k, v, cu, 0.1, **{**dict(seg_base=base, total_rows=rows), **bad})
     with pytest.raises(_lib.WnwError):
         decode_attn(q.float(), k, v, cu, 0.1, seg_base=base, total_rows=rows)
+    with pytest.raises(OverflowError):  # the general path's float(scale)
+        decode_attn(q, k, v, cu, 10**400, seg_base=base, total_rows=rows)
     with pytest.raises(_lib.WnwError, match="group must be"):
         decode_attn(q.repeat(1, 8, 1), k, v, cu, 0.1, seg_base=base, total_rows=rows)
     with pytest.raises(RuntimeError):  # no storage under vmap

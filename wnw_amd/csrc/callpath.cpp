@@ -50,12 +50,16 @@ bool row_major(const at::Tensor& t, int64_t d) {
 bool number(PyObject* o, double* x) {
   if (!PyFloat_CheckExact(o) && !PyLong_CheckExact(o)) return false;
   *x = PyFloat_AsDouble(o);
-  return !(*x == -1.0 && PyErr_Occurred());
+  if (*x != -1.0 || !PyErr_Occurred()) return true;
+  PyErr_Clear();  // beyond the type's range: the general path's to judge
+  return false;
 }
 bool whole(PyObject* o, int64_t* x) {
   if (!PyLong_CheckExact(o)) return false;
   *x = PyLong_AsLongLong(o);
-  return !(*x == -1 && PyErr_Occurred());
+  if (*x != -1 || !PyErr_Occurred()) return true;
+  PyErr_Clear();
+  return false;
 }
 
 struct Ref {  // an owned reference

@@ -23,6 +23,8 @@ def _plain(*tensors: Tensor) -> bool:
     if torch.compiler.is_compiling() or _get_current_dispatch_mode() is not None or forward_ad._current_level >= 0 \
             or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_function_stack() > 0:
         return False
+    if torch.is_autocast_enabled("cuda") and tensors[0].dtype != torch.get_autocast_dtype("cuda"):
+        return False  # the PyTorch form computes in, and returns, autocast's type
     grad = torch.is_grad_enabled()
     return all(type(t) is Tensor and t.is_cuda and t.device == tensors[0].device and not (grad and t.requires_grad)
                for t in tensors)
