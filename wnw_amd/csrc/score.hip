@@ -459,7 +459,7 @@ __global__ __launch_bounds__(kScoreThreads) void seg_score_kernel(SegScoreParams
     for (int u = 0; u < U; ++u) {
       // several short chains of matrix instructions instead of one, so that
       // fewer roundings meet the growing sum: error against 64 bits 7.2e-8 ->
-      // 6.6e-8 (by butterflies 6.7e-8) for 1 % of the time
+      // 6.6-6.8e-8 (by butterflies 6.7-6.8e-8) for 1 % of the time
       f32x4 y[NA];
 #pragma unroll
       for (int n = 0; n < NA; ++n) y[n] = dot_chunk<T>(kb[u][n], qb[n], f32x4{0.f, 0.f, 0.f, 0.f});
