@@ -201,12 +201,14 @@ __device__ __forceinline__ void prev_finish(const AttnParams& p, int tid, const 
 static constexpr int kXlRows = 3;
 
 // A 4-byte copy per lane from a 64-bit address into LDS (lane i's dword at
-// lds_addr + 4 i), counted by vmcnt like the stream's loads.
+// lds_addr + 4 i), counted by vmcnt like the stream's loads.  One wait state
+// between the write of M0 and the load.
 __device__ __forceinline__ void dma_copy4_a64(const void* gaddr, uint32_t lds_addr) {
   uint32_t save;
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
       "global_load_lds_dword %1, off\n\t"
       "s_mov_b32 m0, %0"
       : "=&s"(save)
@@ -1037,12 +1039,18 @@ static constexpr int kSRows = 16;    // rows per step
 
 // 16 bytes per lane from gbase + voff into LDS at lds_addr + 16 * lane.
 // M0 carries the LDS address; it is saved and restored around the load, so
-// the compiler's own uses of M0 are unaffected.
+// the compiler's own uses of M0 are unaffected.  The waits are the ones the
+// compiler puts before such a load of its own: one state between the write of
+// M0 and the load, five between a vector instruction's write of the scalar
+// base (readfirstlane) and the load, two of which the moves are (64 segments of
+// up to 7,564 rows 19.9 -> 20.05 us a launch; longer waits for the first load
+// from a base alone measured no faster).
 __device__ __forceinline__ void dma_copy16(const void* gbase, uint32_t voff, uint32_t lds_addr) {
   uint32_t save;
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %3\n\t"
+      "s_nop 2\n\t"
       "global_load_lds_dwordx4 %1, %2 nt\n\t"
       "s_mov_b32 m0, %0"
       : "=&s"(save)
@@ -1057,6 +1065,7 @@ __device__ __forceinline__ void dma_copy16_a64(const void* gaddr, uint32_t lds_a
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
       "global_load_lds_dwordx4 %1, off nt\n\t"
       "s_mov_b32 m0, %0"
       : "=&s"(save)

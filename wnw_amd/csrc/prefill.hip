@@ -111,12 +111,15 @@ static constexpr int kPaKeys = 64;  // keys per tile
 static constexpr float kPaLag = 8.f;  // log2 of the largest weight before the sums are rescaled
 
 // 16 bytes per lane from gbase + voff into LDS at lds_addr + 16 * lane (M0
-// carries the LDS address and is restored).
+// carries the LDS address and is restored).  One wait state between M0's write
+// and the load, five between a vector instruction's write of the base and the
+// load, the two moves among them.
 __device__ __forceinline__ void prompt_copy16(const void* gbase, uint32_t voff, uint32_t lds_addr) {
   uint32_t save;
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %3\n\t"
+      "s_nop 2\n\t"
       "global_load_lds_dwordx4 %1, %2\n\t"
       "s_mov_b32 m0, %0"
       : "=&s"(save)

@@ -77,12 +77,15 @@ __global__ __launch_bounds__(256) void read_stream_vgpr_kernel(const u32x4* __re
 }
 
 // 16 bytes per lane from gbase + voff into LDS at lds_addr + 16 * lane (M0
-// carries the LDS address and is restored after the load).
+// carries the LDS address and is restored after the load).  One wait state
+// between M0's write and the load, five between a vector instruction's write
+// of the base and the load, the two moves among them.
 __device__ __forceinline__ void ys_dma16(const void* gbase, uint32_t voff, uint32_t lds_addr) {
   uint32_t save;
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %3\n\t"
+      "s_nop 2\n\t"
       "global_load_lds_dwordx4 %1, %2 nt\n\t"
       "s_mov_b32 m0, %0"
       : "=&s"(save)
