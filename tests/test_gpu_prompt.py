@@ -7,6 +7,8 @@ logits of exact 16-bit products, 32-bit sums: 1e-6 + 1e-4 |ref| (weights in
 [0, 1], the exponential's argument error scales with the logits)."""
 import pytest
 import torch
+import torch.nn.functional as F
+from torch.nn.attention import SDPBackend, sdpa_kernel
 
 from wnw_amd import _lib
 from wnw_amd.wnw import prompt, session
@@ -52,10 +54,9 @@ def test_causal_attention_large_scores(gpu):
 @pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 4e-3), (torch.float16, 5e-4)])
 @pytest.mark.parametrize("step", [2.0, 7.5, 8.5])
 def test_causal_attention_rising_scores(gpu, dtype, tol, step):
-    """The weights' reference trails the maximum by up to 8 (log2): scores
-    that rise by less and by more than that from one 64-key tile to the next,
-    and fall again.  A weight's relative rounding does not depend on the
-    reference, so the bounds are the ones above."""
+    """Scores that rise from one 64-key tile to the next, by less and by more
+    than 8 in log2, and fall again: tiles that rescale the sums and tiles that
+    do not."""
     q, k, v = _qkv(gpu, 1, 2, 700, 128, dtype, 11, "heads")
     q[..., 0] = 8.0
     tiles = torch.tensor([0, 1, 2, 3, 3, 4, 2, 5, 0, 6, 7], device=gpu, dtype=torch.float32)
@@ -64,6 +65,24 @@ def test_causal_attention_rising_scores(gpu, dtype, tol, step):
            torch.full((700, 700), float("-inf"), device=gpu, dtype=torch.float64).triu_(1)).softmax(-1) @ v.double()
     out = prompt.causal_attention(q, k, v, 0.08)
     assert float((out.double() - ref).norm() / ref.norm()) < tol
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.float16, 128), (torch.bfloat16, 64),
+                                     (torch.float16, 64)])
+@pytest.mark.parametrize("deviation", [0.5, 1.0, 2.0, 4.0])
+def test_causal_attention_no_less_exact_than_sdpa(gpu, dtype, D, deviation):
+    """Flat to peaked rows against 64 bits, beside SDPA's fused kernels: the
+    same rounding points (the largest weight is 1, 16-bit weights in the value
+    product, 32-bit sums), so errors that differ by the order of the 32-bit sums
+    only.  1 % of a 16-bit rounding is far above that (measured 0.01 %)."""
+    q, k, v = _qkv(gpu, 1, 4, 1111, D, dtype, 21, "heads")
+    q, scale = (q.float() * deviation).to(dtype), D ** -0.5
+    ref = ((q.double() @ k.double().transpose(-1, -2).contiguous()) * scale +
+           torch.full((1111, 1111), float("-inf"), device=gpu, dtype=torch.float64).triu_(1)).softmax(-1) @ v.double()
+    with sdpa_kernel([SDPBackend.FLASH_ATTENTION, SDPBackend.EFFICIENT_ATTENTION]):
+        sdpa = F.scaled_dot_product_attention(q, k, v, is_causal=True, scale=scale)
+    err, theirs = (float((x.double() - ref).norm() / ref.norm()) for x in (prompt.causal_attention(q, k, v, scale), sdpa))
+    assert err <= 1.01 * theirs, (err, theirs)
 
 
 def test_inputs_left_to_torch(gpu):

@@ -81,22 +81,22 @@ struct PromptOps<float> {
 //       keys 8 j + 4 hi + 0..3 of query n, which is already the P^T operand
 //       when V^T's k-slots follow the same order: two ds_read_b64_tr_b16 per
 //       operand (4 keys x 1 column per lane each; V chunks swizzled by 2 (row % 4)).
-// Online softmax in-lane (queries are columns), against a reference that trails
-// the running maximum by up to 2^kPaLag: the sums are rescaled only in tiles
-// where some query's maximum passed that (with 32 queries per wave one of them
-// grows in most of the first 50 tiles; 66 of 207 vector instructions a tile).
-// The weights are then up to 2^8 instead of 1, which their rounding to 16 bits
-// (relative) and the 32-bit sums do not see.  Only the diagonal tile masks, and
-// only the last tile clamps its rows.  P goes through 16 bits, its sum stays
-// 32-bit.
+// Online softmax in-lane (queries are columns) against the running maximum: the
+// sums are rescaled in the tiles where some query's maximum grew (with 32
+// queries per wave most of the first 50).  A row's largest weight is then 1,
+// exact in 16 bits; against a reference that trails the maximum by up to 2^8 it
+// would be rounded beside a sum that is not (178 us instead of 187, error
+// against 64 bits 3 % larger at a standard deviation of the scores of 1, 16 %
+// at 2, 20 % at 4).  Only the diagonal tile masks, and only the last tile clamps
+// its rows.  P goes through 16 bits, its sum stays 32-bit.
 // Bound by the issue of vector instructions (exponentials above all) beside
 // the matrix instructions: two waves per SIMD overlap them only in part.
 // bf16, D = 128, 32 heads: 4,564 rows 588 us (SDPA's flash kernel, 290 TFLOP/s) ->
-// 183 us (933; 202 with every growth rescaled, a mask in every tile and the
-// copies' offsets worked out per tile), 2 x 28 heads of 2,000 rows 85 -> 71 us; the
-// same error against 64 bits.  Measured and not kept: 64 queries per wave and
-// one wave per SIMD (306 us: sums move through accumulator registers), the next
-// tile's scores issued ahead of a tile's softmax (189-190 against 194 us, more
+// 187 us (914; 202 with a mask in every tile and the copies' offsets worked out
+// per tile), 2 x 28 heads of 2,000 rows 85 -> 73 us; SDPA's error against 64 bits
+// to four digits.  Measured and not kept: 64 queries per wave and one wave per
+// SIMD (306 us: sums move through accumulator registers), the next tile's
+// scores issued ahead of a tile's softmax (189-190 against 194 us, more
 // registers), the first values of a tile read ahead of its softmax (the same).
 struct PromptAttnParams {
   const void *q, *k, *v;
@@ -108,7 +108,6 @@ struct PromptAttnParams {
 
 static constexpr int kPaQ = 128;   // queries per workgroup
 static constexpr int kPaKeys = 64;  // keys per tile
-static constexpr float kPaLag = 8.f;  // log2 of the largest weight before the sums are rescaled
 
 // 16 bytes per lane from gbase + voff into LDS at lds_addr + 16 * lane (M0
 // carries the LDS address and is restored).  One wait state between M0's write
@@ -197,7 +196,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PromptAttnParams p
   f32x16 o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) o[dt] = f32x16{};
-  // the reference of the weights: below every score (a fully masked value is -inf)
+  // the running maximum starts below every score (a fully masked value is -inf)
   float m = -3.402823466e38f, l = 0.f;
   const int ntile = min((qblk + 1) * (kPaQ / kPaKeys), (S + kPaKeys - 1) / kPaKeys);
   const int mine = min((q0 + 31) / kPaKeys, ntile - 1);  // the wave's diagonal tile
@@ -225,7 +224,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PromptAttnParams p
 #pragma unroll
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[mt][r]);
     mx = max_x32(mx);
-    if (__ballot((mx - m) * p.scale_log2 > kPaLag)) {
+    if (__ballot(mx > m)) {
       const float alpha = __builtin_amdgcn_exp2f((m - mx) * p.scale_log2);
       l *= alpha;
 #pragma unroll

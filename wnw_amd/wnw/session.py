@@ -77,7 +77,7 @@ def prefill_attention(q: Tensor, k: Tensor, v: Tensor, attention_mask: Tensor | 
 
     Without a mask, GPU inputs in 16 bits run the prompt kernel (head_dim
     64 or 128, nothing to differentiate; 4,564 rows of 32 heads at head_dim
-    128: 211 us against SDPA's 588).  Otherwise SDPA runs with its fused
+    128: 187 us against SDPA's 588).  Otherwise SDPA runs with its fused
     backends only (flash, memory-efficient); when neither takes the inputs,
     the same attention is computed in float32 over query chunks with
     contiguous operands (the products in float32, so no batched bf16 product
