@@ -85,6 +85,21 @@ def test_causal_attention_no_less_exact_than_sdpa(gpu, dtype, D, deviation):
     assert err <= 1.01 * theirs, (err, theirs)
 
 
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.float16, 64)])
+@pytest.mark.parametrize("S", [1, 33, 65, 127, 200, 256])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf")])
+def test_causal_attention_infinite_last_value(gpu, dtype, D, S, value):
+    """An infinity in the last row of V: the last query's output is that
+    infinity, as SDPA gives it, and no query before the row's 64-key tile sees
+    it (within the tile 0 * infinity is NaN there too)."""
+    q, k, v = _qkv(gpu, 1, 2, S, D, dtype, S, "heads")
+    v[:, :, -1, 5] = value
+    out = prompt.causal_attention(q, k, v, 0.1)
+    assert (out[:, :, -1, 5] == value).all()
+    assert torch.isfinite(out[:, :, :(S - 1) // 64 * 64]).all()
+    assert torch.isfinite(torch.cat([out[..., :5], out[..., 6:]], dim=-1)).all()
+
+
 def test_inputs_left_to_torch(gpu):
     q, k, v = _qkv(gpu, 1, 2, 40, 128, torch.bfloat16, 3, "heads")
     assert prompt.causal_attention(q, k, v, 0.1) is not None

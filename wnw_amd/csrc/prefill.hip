@@ -243,13 +243,33 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PromptAttnParams p
         pb[kk][j] = Ops::pack2(x0, x1);
       }
     }
+    // the rows past the prompt repeat its last one: their weights are 0, and V
+    // is made 0 too (an infinity there would give NaN with them)
+    uint64_t vm[4][2];
+    const int end = p.S - i * kPaKeys;  // keys of the prompt in this tile
+    bool cut = false;
+    if constexpr (decltype(masked)::value) {
+      cut = end < kPaKeys;
+      if (cut)
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int left = end - (16 * kk + 8 * j + 4 * hi);  // of the lane's 4 keys
+            vm[kk][j] = left <= 0 ? 0 : left >= 4 ? ~0ull : (1ull << (16 * left)) - 1;
+          }
+    }
     __builtin_amdgcn_s_setprio(1);  // a wave at its products before another's softmax: 185 -> 183 us
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
-        const uint64_t v0 = Ops::read_tr(vt + voff[dt] + 16 * kk * RB);
-        const uint64_t v1 = Ops::read_tr(vt + voff[dt] + (16 * kk + 8) * RB);
+        uint64_t v0 = Ops::read_tr(vt + voff[dt] + 16 * kk * RB);
+        uint64_t v1 = Ops::read_tr(vt + voff[dt] + (16 * kk + 8) * RB);
+        if (cut) {
+          v0 &= vm[kk][0];
+          v1 &= vm[kk][1];
+        }
         const u32x4 a = u32x4{(uint32_t)v0, (uint32_t)(v0 >> 32), (uint32_t)v1, (uint32_t)(v1 >> 32)};
         o[dt] = Ops::mma32(a, pb[kk], o[dt]);
       }
