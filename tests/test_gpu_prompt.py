@@ -121,6 +121,25 @@ def test_inputs_left_to_torch(gpu):
     torch.testing.assert_close(got[0], session.prefill_attention(q, k, v, None, 0.1), atol=2e-2, rtol=2e-2)
 
 
+def test_traced_programs_record_torch_operators(gpu):
+    """torch.jit.trace sees operators only: a launch behind its back would
+    leave the traced program with unwritten memory."""
+    q, k, v = _qkv(gpu, 1, 4, 96, 128, torch.bfloat16, 3, "heads")
+    q2 = _qkv(gpu, 1, 4, 96, 128, torch.bfloat16, 4, "heads")[0]
+    traced = torch.jit.trace(lambda a, b, c: session.prefill_attention(a, b, c, None, 0.1), (q, k, v), check_trace=False)
+    want = session.prefill_attention(q2, k, v, None, 0.1)
+    torch.testing.assert_close(traced(q2, k, v), want, atol=2e-2, rtol=2e-2)
+    cache = _Cache(_Config([0], 2, "mean_text"), [2], [90])
+
+    def scores(a, b):
+        class_a, per_head = session.compute_prefill_scores(a, b, None, cache, 0, 2, 2, 0.1)
+        return class_a[0], per_head[0][1]
+
+    traced = torch.jit.trace(scores, (q, k[:, :2]), check_trace=False)
+    for x, y in zip(traced(q2, k[:, :2]), scores(q2, k[:, :2])):
+        torch.testing.assert_close(x, y, atol=1e-3, rtol=2e-2)
+
+
 class _Config:
     def __init__(self, a_heads, group, mode):
         self.prefill_score_mode, self._a, self._g = mode, a_heads, group

@@ -27,3 +27,13 @@ def test_prefill_attention_fallback_matches_sdpa(mask, monkeypatch):
     monkeypatch.setattr(session.F, "scaled_dot_product_attention", no_fused_backend)
     got = session.prefill_attention(q, k, v, m, 0.3, q_chunk=10)
     torch.testing.assert_close(got, want, atol=2e-6, rtol=1e-5)
+
+
+def test_prefill_attention_under_tracers():
+    """A symbolic trace and a compiled graph record SDPA, for any inputs."""
+    q, k, v = (torch.randn(1, 2, 24, 64) for _ in range(3))
+    want = session.prefill_attention(q, k, v, None, 0.3)
+    traced = torch.fx.symbolic_trace(session.prefill_attention, concrete_args={"attention_mask": None, "scaling": 0.3})
+    torch.testing.assert_close(traced(q, k, v, None, 0.3), want)
+    compiled = torch.compile(session.prefill_attention, backend="eager")
+    torch.testing.assert_close(compiled(q, k, v, None, 0.3), want)

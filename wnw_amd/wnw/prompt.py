@@ -19,15 +19,17 @@ from .. import _lib
 
 def _plain(*tensors: Tensor) -> bool:
     """GPU tensors that nothing traces, transforms or differentiates: the
-    kernels write their results behind autograd's back."""
-    if torch.compiler.is_compiling() or _get_current_dispatch_mode() is not None or forward_ad._current_level >= 0 \
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_function_stack() > 0:
+    kernels write their results behind autograd's back.  To be asked before
+    anything else of the tensors, which may be a symbolic tracer's."""
+    if torch.compiler.is_compiling() or any(type(t) is not Tensor for t in tensors):
+        return False
+    if torch._C._get_tracing_state() is not None or _get_current_dispatch_mode() is not None \
+            or forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_function_stack() > 0:
         return False
     if torch.is_autocast_enabled("cuda") and tensors[0].dtype != torch.get_autocast_dtype("cuda"):
         return False  # the PyTorch form computes in, and returns, autocast's type
     grad = torch.is_grad_enabled()
-    return all(type(t) is Tensor and t.is_cuda and t.device == tensors[0].device and not (grad and t.requires_grad)
-               for t in tensors)
+    return all(t.is_cuda and t.device == tensors[0].device and not (grad and t.requires_grad) for t in tensors)
 
 
 def _rows_ok(*tensors: Tensor) -> bool:
@@ -43,9 +45,9 @@ def causal_attention(q: Tensor, k: Tensor, v: Tensor, scaling: float) -> Tensor 
     """Causal attention [B, H, S, D] of equally long q, k, v (bf16 / f16,
     head_dim 64 or 128), the result with q's strides, as SDPA's fused
     kernels return it."""
-    if not (q.dim() == 4 and q.shape == k.shape == v.shape and q.dtype == k.dtype == v.dtype
+    if not (_plain(q, k, v) and q.dim() == 4 and q.shape == k.shape == v.shape and q.dtype == k.dtype == v.dtype
             and q.dtype in (torch.bfloat16, torch.float16) and q.shape[3] in (64, 128) and q.numel() > 0
-            and scaling > 0 and _plain(q, k, v)):
+            and scaling > 0):
         return None
     out = torch.empty_like(q)
     if not _rows_ok(q, k, v, out) or max(t.stride(2) for t in (q, k, v, out)) > 1 << 22:
@@ -66,6 +68,9 @@ def token_scores(q: Tensor, k: Tensor, attention_mask: Tensor | None, audio_star
     (``wnw_prefill_scores``): per sample the class-A heads' row (None
     without class-A heads) and one row per entry of ``kv_heads``.
     ``attention_mask``: additive [B, 1, S, S], or None for causal."""
+    m = attention_mask
+    if not _plain(*((q, k) if m is None else (q, k, m))):
+        return None
     if not (q.dim() == k.dim() == 4 and q.dtype == k.dtype and q.dtype in _lib._TORCH_DTYPES
             and q.shape[0] == k.shape[0] and q.shape[2:] == k.shape[2:] and q.shape[3] in (64, 128, 256)
             and q.shape[1] == k.shape[1] * group and q.numel() > 0):
@@ -75,10 +80,9 @@ def token_scores(q: Tensor, k: Tensor, attention_mask: Tensor | None, audio_star
             any(not (0 <= a < e <= S) for a, e in zip(audio_starts, audio_ends)) or \
             any(not 0 <= h < q.shape[1] for h in class_a_heads) or any(not 0 <= h < k.shape[1] for h in kv_heads):
         return None
-    m = attention_mask
     if m is not None and not (m.dtype in _lib._TORCH_DTYPES and m.shape == (B, 1, S, S) and m.stride(3) == 1):
         return None
-    if not _plain(*((q, k) if m is None else (q, k, m))) or not _rows_ok(q, k):
+    if not _rows_ok(q, k):
         return None
     dev = q.device
     width = max(e - a for a, e in zip(audio_starts, audio_ends))
