@@ -316,21 +316,49 @@ struct SegScoreParams {
 
 // 16 rows x 16 heads of q . K: A = the rows' 16-byte chunks, B = q's, lane
 // (lq, lc) = (lane / 16, lane % 16) holding chunk 4 c + lq of row / head lc;
-// the sum's lane holds rows 4 lq + i of head lc.  16-bit products are exact in
-// the 32-bit sums, and fp32 runs on 32-bit matrix operands.
-template <typename T>
-__device__ __forceinline__ f32x4 dot_chunk(const u32x4& a, const u32x4& b, f32x4 c) {
+// the sum's lane holds rows 4 lq + i of head lc.  Every matrix instruction
+// (32 exact 16-bit products, or 4 fp32 ones) starts from zero and the results
+// are added pairwise, N of them from number LO on, so that no rounding meets
+// more of the sum than in a tree of short scalar chains: error of a dot of 128
+// over its size 4.7e-8 in bf16, 7.3e-8 in fp32 (as one chain 6.0e-8 and 2.0e-7,
+// as four 4.7e-8 and 1.1e-7; a tree of chains of 8 / 4 fused multiply-adds
+// 4.8e-8 and 7.3e-8).  8 items of 7,564 rows, 4 heads, D = 128, both passes: bf16
+// 12.3 us either way, fp32 17.5 -> 19.0 us.
+template <typename T, int LO, int N>
+__device__ __forceinline__ f32x4 dot_tree(const u32x4* a, const u32x4* b) {
+  const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (N > 1)
+    return dot_tree<T, LO, N / 2>(a, b) + dot_tree<T, LO + N / 2, N / 2>(a, b);
+  else if constexpr (sizeof(T) == 4)
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[LO / 4][LO % 4]), __uint_as_float(b[LO / 4][LO % 4]),
+                                                zero, 0, 0, 0);
+  else if constexpr (std::is_same<T, bf16_t>::value)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[LO]), __builtin_bit_cast(bf16x8, b[LO]),
+                                                   zero, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a[LO]), __builtin_bit_cast(f16x8, b[LO]),
+                                                  zero, 0, 0, 0);
+}
+// The dots of NC chunks.  fp32: 8 results at a time, ordered by passing the
+// next chunks through an empty instruction that takes the last 8's sum (all
+// 64 at D = 256 at once would leave one wave per SIMD, and that one spilling).
+template <typename T, int NC>
+__device__ __forceinline__ f32x4 dot_rows(u32x4* a, const u32x4* b) {
   if constexpr (sizeof(T) == 4) {
+    constexpr int NG = NC / 2;
+    f32x4 y[NG];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[j]), __uint_as_float(b[j]), c, 0, 0, 0);
-    return c;
-  } else if constexpr (std::is_same<T, bf16_t>::value) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
-                                                   0, 0);
+    for (int g = 0; g < NG; ++g) {
+      if (g > 0) asm volatile("" : "+v"(a[2 * g]), "+v"(a[2 * g + 1]) : "v"(y[g - 1]));
+      y[g] = dot_tree<T, 0, 8>(a + 2 * g, b + 2 * g);
+    }
+#pragma unroll
+    for (int o = 1; o < NG; o *= 2)
+#pragma unroll
+      for (int g = 0; g + o < NG; g += 2 * o) y[g] += y[g + o];
+    return y[0];
   } else {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
-                                                  0);
+    return dot_tree<T, 0, NC>(a, b);
   }
 }
 
@@ -376,7 +404,6 @@ __global__ __launch_bounds__(kScoreThreads) void seg_score_kernel(SegScoreParams
   constexpr int EPC = RowGeom<T>::EPC;
   constexpr int NC = D / EPC / 4;           // chunks of a row per lane
   constexpr int U = NC >= 8 ? 1 : 8 / NC;   // tiles whose loads are in flight per wave
-  constexpr int NA = NC < 4 ? NC : 4;       // sums of a dot, added pairwise
   constexpr int NW = kScoreThreads / 64;
   __shared__ float stat[kMaxHeads][2];
   __shared__ float red[SCORE ? 1 : NW][kMaxHeads][2];
@@ -456,21 +483,7 @@ __global__ __launch_bounds__(kScoreThreads) void seg_score_kernel(SegScoreParams
   for (int t0 = w; t0 < ntiles; t0 += NW * U) {
     f32x4 x[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      // several short chains of matrix instructions instead of one, so that
-      // fewer roundings meet the growing sum: error against 64 bits 7.2e-8 ->
-      // 6.6-6.8e-8 (by butterflies 6.7-6.8e-8) for 1 % of the time
-      f32x4 y[NA];
-#pragma unroll
-      for (int n = 0; n < NA; ++n) y[n] = dot_chunk<T>(kb[u][n], qb[n], f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-      for (int n = NA; n < NC; ++n) y[n % NA] = dot_chunk<T>(kb[u][n], qb[n], y[n % NA]);
-#pragma unroll
-      for (int o = 1; o < NA; o *= 2)
-#pragma unroll
-        for (int n = 0; n + o < NA; n += 2 * o) y[n] += y[n + o];
-      x[u] = y[0];
-    }
+    for (int u = 0; u < U; ++u) x[u] = dot_rows<T, NC>(kb[u], qb);
     if (t0 + NW * U < ntiles) load(t0 + NW * U);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -479,7 +492,7 @@ __global__ __launch_bounds__(kScoreThreads) void seg_score_kernel(SegScoreParams
         float sc[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          sc[i] = lc < nh ? exp2f(x[u][i] * p.scale_log2 - m) * l : 0.f;
+          sc[i] = lc < nh ? exp2f(fmaf(x[u][i], p.scale_log2, -m)) * l : 0.f;
           // the 16 heads of the lane's row group
 #pragma unroll
           for (int o = 8; o >= 1; o >>= 1) sc[i] += __shfl_xor(sc[i], o);
@@ -490,15 +503,13 @@ __global__ __launch_bounds__(kScoreThreads) void seg_score_kernel(SegScoreParams
           *a += mine;
         }
       } else {
-        float v[4], mx = m;
+        // the scaled dot enters the exponent unrounded, as it does in the scores
+        float mx = m;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          v[i] = row + i < c1 ? x[u][i] * p.scale_log2 : -INFINITY;
-          mx = fmaxf(mx, v[i]);
-        }
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, row + i < c1 ? x[u][i] * p.scale_log2 : -INFINITY);
         l *= exp2f(m - mx);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) l += exp2f(v[i] - mx);
+        for (int i = 0; i < 4; ++i) l += row + i < c1 ? exp2f(fmaf(x[u][i], p.scale_log2, -mx)) : 0.f;
         m = mx;
       }
     }
