@@ -68,3 +68,34 @@ def test_two_level_merge(gpu, dtype, G, D, n_wg):
         got, ref = _run_case(gpu, lens, G, D, dtype, n_wg=n_wg, seed=seed)
         ok, msg = allclose_report(got, ref, *_tol(dtype))
         assert ok, msg
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("G", [4, 16])
+@pytest.mark.parametrize("nats", [12.0, 17.5, 20.0])
+def test_weights_in_32_bits_beside_a_sink(gpu, dtype, G, nats):
+    """head_dim 256, one workgroup: a row whose V is zero and whose score is far
+    above the others', so that the output is made of weights of 6e-6 to 2e-9
+    of the maximum, below what f16 holds.  Bound: the output's own rounding
+    (2^-11 / 2^-8, in 2-norm 0.3 to 0.6 of that) and the 32-bit sums."""
+    import torch
+
+    from wnw_amd.kv.fused_attn import decode_attn
+
+    n, D, dt = 6000, 256, getattr(torch, dtype)
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(int(nats))
+    k = torch.randn(n, D, device=gpu, generator=gen) * 0.05
+    k[:, 0] = 0
+    k[3, 0] = nats
+    v = torch.rand(n, D, device=gpu, generator=gen) + 0.5
+    v[3] = 0
+    v *= 2.0 ** min(14, round(nats * 1.4427 - 12.5))  # the output in the range of normal f16
+    q = torch.randn(1, G, D, device=gpu, generator=gen) * 0.1
+    q[..., 0] = 16.0
+    q, k, v = q.to(dt), k.to(dt), v.to(dt)
+    ref = ((q[0].double() @ k.double().t()) / 16).softmax(-1) @ v.double()
+    cu = torch.tensor([0, n], dtype=torch.int32, device=gpu)
+    out = decode_attn(q, k, v, cu, 1 / 16, n_wg=1)[0].double()
+    err = float((out - ref).norm() / ref.norm())
+    assert err < (4e-4 if dtype == "float16" else 3e-3), err

@@ -1010,7 +1010,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_mfma_kernel(AttnParams p) {
 // (MI355X, per launch): fp32 D = 128, G = 4, 5,632 rows 74.8 -> 14.2 us (the
 // VALU kernel read each lane's own row, 512 bytes apart, one step at a time;
 // the separate append launch of 4.8 us is gone too); bf16 D = 256, G = 4,
-// 35 MB 106.7 -> 24.5 us; fp16 D = 128, G = 16, 40 MB 43.0 -> 32.4 us (MFMA
+// 35 MB 106.7 -> 27.0 us; fp16 D = 128, G = 16, 40 MB 43.0 -> 32.4 us (MFMA
 // kernel: V transposed by 16-bit LDS reads).
 //
 // Each wave owns a contiguous quarter of its workgroup's row range and walks
@@ -1025,7 +1025,10 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_mfma_kernel(AttnParams p) {
 //   S^T (16 rows x 16 heads) = K_tile x q^T: D/32 v_mfma_f32_16x16x32, the
 //       K operand read row by row from LDS (16-byte chunks XOR-swizzled by
 //       the row, so the 16 rows of one read hit distinct banks);
-//   (fp32: v_mfma_f32_16x16x4_f32, 32-bit operands and sums throughout)
+//   (fp32: v_mfma_f32_16x16x4_f32, 32-bit operands and sums throughout;
+//   16-bit rows of 256: that instruction for O^T, weights kept in 32 bits and
+//   V widened, since a 16-bit pair drops f16 weights below 2^-25 of a wave's
+//   largest, and inf * (hi + lo) is NaN: 23.4 -> 27.0 us at 35 MB)
 //   O^T += V^T x P^T: D/16 tiles of v_mfma_f32_16x16x16, two per tile (P
 //       split into hi + lo halves); the V^T operand comes from one
 //       ds_read_b64_tr_b16 per lane and tile (4 rows x 1 column each),
@@ -1277,6 +1280,7 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
   constexpr int kSaveRows = stream_save_rows(G_::RB);
   constexpr int kHeads = stream_heads(QD);
   constexpr bool kF32 = sizeof(T) == 4;
+  constexpr bool kP32 = kF32 || D > 128;  // 32-bit weights in the value product
   constexpr int NT = NW * 64;
   constexpr int RB = G_::RB, SB = G_::SB, NI = G_::NI, RPI = G_::RPI, CH = G_::CH, NC = G_::NC, NTD = G_::NTD;
   constexpr int QX = QD + (APPEND ? 1 : 0);  // first-step loads besides K and V: q (and the new row)
@@ -1316,8 +1320,9 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
   const T* kp = (const T*)p.k;
   const T* vp = (const T*)p.v;
   // rows [row0, row0 + nrows) of K or V into step buffer b, 16-byte chunks
-  // swizzled by the row (K: chunk ^ (r % CH); V: chunk ^ 2 (r % 4), fp32 V
-  // not at all); rows past nrows repeat the last row
+  // swizzled by the row (K: chunk ^ (r % CH); V: chunk ^ v_swizzle(r)); rows
+  // past nrows repeat the last row
+  auto v_swizzle = [](int r) { return kF32 ? 0 : kP32 ? 8 * ((r >> 2) & 1) : 2 * (r & 3); };
   auto load_rows = [&](bool is_v, int64_t row0, int nrows, int b) {
     // wave-uniform addresses, kept scalar (the load takes them in SGPRs)
     const T* src = (const T*)uni((int64_t)(uintptr_t)((is_v ? vp : kp) + row0 * D));
@@ -1327,7 +1332,7 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
     for (int u = 0; u < NI; ++u) {
       const int r = u * RPI + lane / CH;
       const int rr = max(0, r < nrows ? r : nrows - 1);
-      const int sw = is_v ? (kF32 ? 0 : 2 * (r & 3)) : r % CH;
+      const int sw = is_v ? v_swizzle(r) : r % CH;
       dma_copy16(src, (uint32_t)(rr * RB + (((lane % CH) ^ sw) * 16)), dst + u * 1024);
     }
   };
@@ -1551,9 +1556,9 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
   u32x4 qb[NC];
   // the n-th group of four consecutive elements of head lc that a lane's
   // tiles hold (n < NTD), and its first element's index
-  auto quad_at = [&](int n) { return kF32 ? 64 * (n >> 2) + 16 * lq + 4 * (n & 3) : 16 * n + 4 * lq; };
+  auto quad_at = [&](int n) { return kP32 ? 64 * (n >> 2) + 16 * lq + 4 * (n & 3) : 16 * n + 4 * lq; };
   auto quad = [&](const f32x4* a, int n) -> f32x4 {
-    if constexpr (kF32) {
+    if constexpr (kP32) {
       const int u = n & ~3, i = n & 3;
       return f32x4{a[u][i], a[u + 1][i], a[u + 2][i], a[u + 3][i]};
     }
@@ -1663,9 +1668,10 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
       pv[i] = __builtin_amdgcn_exp2f(x[i] - m_new);
       psum += pv[i];
     }
-    // P = hi + lo, each a 16-bit float: PV runs as two MFMAs with fp32-grade P
+    // P = hi + lo, each a 16-bit float: PV runs as two MFMAs with ~16 (bf16) to
+    // ~22 bits (f16, down to 2^-25 of the wave's maximum) of P
     uint64_t ph = 0, pl = 0;
-    if constexpr (!kF32) {
+    if constexpr (!kP32) {
       const uint32_t h01 = Ops::pack2(pv[0], pv[1]), h23 = Ops::pack2(pv[2], pv[3]);
       const uint32_t l01 = Ops::pack2(pv[0] - Ops::to_f32(h01 & 0xffffu), pv[1] - Ops::to_f32(h01 >> 16));
       const uint32_t l23 = Ops::pack2(pv[2] - Ops::to_f32(h23 & 0xffffu), pv[3] - Ops::to_f32(h23 >> 16));
@@ -1686,23 +1692,36 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
     __builtin_amdgcn_sched_barrier(0);
     if (add_row && lane < CH) {  // the new row's V chunks as row nrows
       const uint8_t* nrow = qbuf + st.qslot * qslot + qarea;
-      *(u32x4*)(vbuf + st.nrows * RB + ((lane ^ (kF32 ? 0 : 2 * (st.nrows & 3))) * 16)) =
+      *(u32x4*)(vbuf + st.nrows * RB + ((lane ^ v_swizzle(st.nrows)) * 16)) =
           *(const u32x4*)(nrow + RB + lane * 16);
     }
     // V^T operand of tile t: lane (lq, lc) addresses row 4 lq + lc / 4, columns
     // 16 t + 4 (lc % 4) .. + 3 (8 bytes of the swizzled row)
-    if constexpr (kF32) {
-      // fp32: k-step i sums rows 4 lq' + i over the lane quarters lq', so the
-      // lane's own p[i] is the P^T operand; tile 4 u + j holds columns 64 u +
-      // 4 m + j (m = 0..15), so one 16-byte read of a row feeds four tiles
+    if constexpr (kP32) {
+      // 32-bit products: k-step i sums rows 4 lq' + i over the lane quarters
+      // lq', so the lane's own p[i] is the P^T operand; tile 4 u + j holds
+      // columns 64 u + 4 m + j (m = 0..15), so one read of 4 elements of a row
+      // feeds four tiles (16 bits: widened here; the swizzle puts two quarters'
+      // 128 bytes in different halves of the banks)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int u = 0; u < NTD / 4; ++u) {
-          const u32x4 a = *(const u32x4*)(vbuf + (4 * lq + i) * RB + (16 * u + lc) * 16);
+          const uint8_t* row = vbuf + (4 * lq + i) * RB;
+          float a[4];
+          if constexpr (kF32) {
+            const u32x4 w4 = *(const u32x4*)(row + (16 * u + lc) * 16);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) a[j] = __uint_as_float(w4[j]);
+          } else {
+            typedef uint32_t u32x2_v __attribute__((ext_vector_type(2)));
+            const u32x2_v w2 = *(const u32x2_v*)(row + ((8 * u + (lc >> 1)) ^ v_swizzle(4 * lq)) * 16 + (lc & 1) * 8);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) a[j] = Ops::to_f32(j & 1 ? w2[j >> 1] >> 16 : w2[j >> 1] & 0xffffu);
+          }
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            acc[4 * u + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[j]), pv[i], acc[4 * u + j], 0, 0, 0);
+            acc[4 * u + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], pv[i], acc[4 * u + j], 0, 0, 0);
         }
     } else {
       const int r = 4 * lq + (lc >> 2);
@@ -1726,11 +1745,13 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
         if (lc < G) {
           [[maybe_unused]] WNW_GLOBAL uint16_t* o = gptr_w<uint16_t>(p.out) + ((int64_t)st.s * G + lc) * D;
           const float inv = 1.f / l_tot;
-          if constexpr (kF32) {
+          if constexpr (kP32) {
 #pragma unroll
-            for (int t = 0; t < NTD; ++t)
-              *(WNW_GLOBAL f32x4*)(gptr_w<float>(p.out) + ((int64_t)st.s * G + lc) * D + quad_at(t)) =
-                  quad(acc, t) * inv;
+            for (int t = 0; t < NTD; ++t) {
+              const f32x4 x = quad(acc, t) * inv;
+              const float o4[4] = {x[0], x[1], x[2], x[3]};
+              store_quad<T>(p.out, ((int64_t)st.s * G + lc) * D + quad_at(t), o4);
+            }
           } else
 #pragma unroll
           for (int t = 0; t < NTD; ++t) {
