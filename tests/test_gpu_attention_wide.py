@@ -99,3 +99,38 @@ def test_weights_in_32_bits_beside_a_sink(gpu, dtype, G, nats):
     out = decode_attn(q, k, v, cu, 1 / 16, n_wg=1)[0].double()
     err = float((out - ref).norm() / ref.norm())
     assert err < (4e-4 if dtype == "float16" else 3e-3), err
+
+
+@pytest.mark.parametrize("dtype,G,D", [("float32", 4, 64), ("float32", 16, 128), ("bfloat16", 4, 256),
+                                       ("float16", 16, 256)])
+@pytest.mark.parametrize("append", [False, True])
+def test_infinite_values(gpu, dtype, G, D, append):
+    """An infinity in V's last row of a segment (the step's rows after it are
+    copies of it, with weight 0) or in the row before it: the output is that
+    infinity, in its column alone."""
+    import torch
+
+    from wnw_amd.kv.fused_attn import decode_attn
+
+    lens, dt = [1, 17, 200, 33, 16, 5], getattr(torch, dtype)
+    n, cap = len(lens), [x + 1 for x in lens]
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(6)
+    rnd = lambda *s: torch.randn(*s, device=gpu, generator=gen)  # noqa: E731
+    base = [sum(cap[:i]) for i in range(n)]
+    q, k, v = rnd(n, G, D).to(dt), rnd(sum(cap), D).to(dt), rnd(sum(cap), D).to(dt)
+    new_k, new_v = rnd(n, D).to(dt), rnd(n, D).to(dt)
+    last = [b + x - 1 for b, x in zip(base, lens)]
+    v[last[2], 9], v[last[3], 3], v[last[1] - 1, 4], v[last[5], 0] = float("inf"), float("-inf"), float("inf"), float("inf")
+    if append:
+        new_v[4, 7] = float("-inf")
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=gpu)  # noqa: E731
+    cu = i32([0] + lens).cumsum(0).to(torch.int32)
+    want = torch.zeros(n, D, device=gpu)
+    want[2, 9], want[3, 3], want[1, 4], want[5, 0] = float("inf"), float("-inf"), float("inf"), float("inf")
+    want[4, 7] = float("-inf") if append else 0
+    app = (new_k, new_v, torch.empty_like(cu), i32(cap)) if append else None
+    for rows in (sum(lens) + n, 64):  # several workgroups and one
+        out = decode_attn(q, k.clone(), v.clone(), cu, 0.05, seg_base=torch.tensor(base, device=gpu), total_rows=rows,
+                          append=app).float()
+        assert torch.equal(torch.where(torch.isfinite(out), 0.0, out), want[:, None].expand_as(out))

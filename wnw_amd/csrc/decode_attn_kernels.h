@@ -1695,6 +1695,13 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
       *(u32x4*)(vbuf + st.nrows * RB + ((lane ^ v_swizzle(st.nrows)) * 16)) =
           *(const u32x4*)(nrow + RB + lane * 16);
     }
+    // rows past the step's repeat its last one; V is made 0 there, because an
+    // infinity in that row times their weight 0 is NaN
+    if constexpr (kP32) {
+      if (nvalid < kSRows)  // wave-uniform
+        for (int r = nvalid + lane / CH; r < kSRows; r += 64 / CH)
+          *(u32x4*)(vbuf + r * RB + (lane % CH) * 16) = u32x4{0, 0, 0, 0};
+    }
     // V^T operand of tile t: lane (lq, lc) addresses row 4 lq + lc / 4, columns
     // 16 t + 4 (lc % 4) .. + 3 (8 bytes of the swizzled row)
     if constexpr (kP32) {
