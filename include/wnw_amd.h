@@ -691,27 +691,29 @@ int wnw_prefill_attn(const void* q, const void* k, const void* v, int64_t batch,
 
 /*
  * Prompt token scores of one layer (src/algorithms/wnw/code/session.py:
- * 119-170), two launches.  q [batch, heads, seq, head_dim], k [batch,
- * kv_heads, seq, head_dim]; strides: element strides (batch, head, row) of q
- * and k (multiples of 16 bytes, head_dim contiguous), then (batch, row) of
- * mask, an additive [batch, 1, seq, seq] of mask_dtype with contiguous rows,
- * or null: causal.  With w the softmax over all keys of scale * q . k + mask
- * and [audio_starts[b], audio_ends[b]) each sample's audio rows (host arrays):
+ * 119-170), two launches.  q [batch, n_heads, seq, head_dim], k [batch,
+ * n_kv_heads, seq, head_dim], group = n_heads / n_kv_heads; strides: element
+ * strides (batch, head, row) of q and k (not negative, multiples of 16 bytes,
+ * head_dim contiguous), then (batch, row) of mask (not negative), an additive
+ * [batch, 1, seq, seq] of mask_dtype with contiguous rows, or null: causal.
+ * With w the softmax over all keys of scale * q . k + mask and
+ * [audio_starts[b], audio_ends[b]) each sample's audio rows (host arrays):
  *   out_a[b, j] = sum over the n_a heads a_heads (against KV head a_heads[0] /
  *       group) of the last row's w at audio row j;
  *   out_h[b, i, j] = sum over the heads of KV head kv_heads[i] of w at audio
  *       row j, of the last row (last_row != 0) or averaged over the rows after
  *       the audio (0 where there are none).
- * max_audio: row length of out_a / out_h; max_queries >= group x rows of any
- * sample and n_a.  head_dim 64, 128 or 256, at most 64 samples, class-A heads
- * and KV heads (WNW_ENOTSUP otherwise).
+ * a_heads lie in [0, n_heads), kv_heads in [0, n_kv_heads).  max_audio: row
+ * length of out_a / out_h; max_queries >= group x rows of any sample and n_a.
+ * head_dim 64, 128 or 256, at most 64 samples, class-A heads and KV heads
+ * (WNW_ENOTSUP otherwise).
  */
 int64_t wnw_prefill_scores_workspace_bytes(int64_t batch, int64_t n_items,
                                            int64_t seq, int64_t head_dim,
                                            int64_t max_queries, int dtype);
 int wnw_prefill_scores(const void* q, const void* k, const void* mask,
-                       const int64_t* strides, int64_t batch, int64_t group,
-                       int64_t seq, int64_t head_dim,
+                       const int64_t* strides, int64_t batch, int64_t n_heads,
+                       int64_t n_kv_heads, int64_t seq, int64_t head_dim,
                        const int32_t* audio_starts, const int32_t* audio_ends,
                        const int32_t* a_heads, int64_t n_a,
                        const int32_t* kv_heads, int64_t n_kv, int last_row,

@@ -43,3 +43,26 @@ def test_host_only_queries_work_without_gpu():
     ws = l.wnw_decode_attn_workspace_bytes(64, 4, 128)
     assert ws > 0 and ws % 256 == 0
     assert l.wnw_decode_attn_workspace_bytes(64, 0, 128) == -1
+
+
+def test_prefill_scores_refuses_reads_outside_its_tensors():
+    """Heads outside the counts, negative strides and sizes beyond the
+    kernel's are refused before anything is launched (the pointers are not
+    looked at)."""
+    good = dict(heads=8, kv_heads=2, a=[0, 7], kv=[1], strides=[65536, 8192, 128, 16384, 8192, 128, 4096, 64],
+                most=256)
+
+    def call(**change):
+        c = {**good, **change}
+        i32 = lambda x: (ctypes.c_int32 * len(x))(*x)  # noqa: E731
+        p = ctypes.c_void_p(1 << 20)
+        return _lib.lib().wnw_prefill_scores(
+            p, p, p, (ctypes.c_int64 * 8)(*c["strides"]), 1, c["heads"], c["kv_heads"], 64, 128, i32([2]), i32([50]),
+            i32(c["a"]), len(c["a"]), i32(c["kv"]), len(c["kv"]), 0, 0.1, _lib.DT_BF16, _lib.DT_BF16, 48, c["most"], p, p,
+            p, 1 << 60, None)
+
+    for i in range(8):
+        assert call(strides=[-x if j == i else x for j, x in enumerate(good["strides"])]) == _lib.WNW_EINVAL
+    for bad in (dict(a=[0, 8]), dict(a=[-1]), dict(kv=[2]), dict(kv=[0, -1]), dict(heads=7), dict(kv_heads=0),
+                dict(heads=0), dict(most=1 << 31)):
+        assert call(**bad) == _lib.WNW_EINVAL, bad

@@ -63,7 +63,7 @@ _SIGNATURES = {
     "wnw_score_kept_logits": (_i32, [_vp, _vp, _vp, _vp] + [_i64] * 4 + [_vp, _vp, _i64, _vp, _vp, _i64, _vp]),
     "wnw_prefill_attn": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp, _f32, _i32, _vp, _vp]),
     "wnw_prefill_scores_workspace_bytes": (_i64, [_i64] * 5 + [_i32]),
-    "wnw_prefill_scores": (_i32, [_vp] * 4 + [_i64] * 4 + [_vp, _vp, _vp, _i64, _vp, _i64, _i32, _f32, _i32, _i32, _i64,
+    "wnw_prefill_scores": (_i32, [_vp] * 4 + [_i64] * 5 + [_vp, _vp, _vp, _i64, _vp, _i64, _i32, _f32, _i32, _i32, _i64,
                                                          _i64, _vp, _vp, _vp, _i64, _vp]),
     "wnw_read_stream": (_i32, [_vp, _i64, _i64, _i32, _vp, _vp]),
     # host planner (CPU only)

@@ -67,7 +67,7 @@ int device_cus() {
 
 extern "C" const char* wnw_last_error(void) { return wnw::g_err; }
 
-extern "C" int wnw_abi_version(void) { return 1; }
+extern "C" int wnw_abi_version(void) { return 2; }
 
 extern "C" int wnw_init(void) {
   int32_t* w = wnw::device_error_word();

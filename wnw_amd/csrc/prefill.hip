@@ -606,7 +606,8 @@ extern "C" int64_t wnw_prefill_scores_workspace_bytes(int64_t batch, int64_t n_i
 }
 
 extern "C" int wnw_prefill_scores(const void* q, const void* k, const void* mask, const int64_t* strides, int64_t batch,
-                                  int64_t group, int64_t seq, int64_t head_dim, const int32_t* audio_starts,
+                                  int64_t n_heads, int64_t n_kv_heads, int64_t seq, int64_t head_dim,
+                                  const int32_t* audio_starts,
                                   const int32_t* audio_ends, const int32_t* a_heads, int64_t n_a,
                                   const int32_t* kv_heads, int64_t n_kv, int last_row, float scale, int dtype,
                                   int mask_dtype, int64_t max_audio, int64_t max_queries, float* out_a, float* out_h,
@@ -616,9 +617,12 @@ extern "C" int wnw_prefill_scores(const void* q, const void* k, const void* mask
     set_error("the prompt scores take up to %d samples, class-A heads and KV heads, head_dim 64, 128 or 256", kPsMax);
     return WNW_ENOTSUP;
   }
-  WNW_CHECK_ARG(batch >= 0 && group >= 1 && seq >= 0 && seq < (1ll << 30) && n_a >= 0 && n_kv >= 0 && max_audio >= 0 &&
-                    max_queries >= 0,
+  WNW_CHECK_ARG(batch >= 0 && seq >= 0 && seq < (1ll << 30) && n_a >= 0 && n_kv >= 0 && max_audio >= 0 &&
+                    max_queries >= 0 && max_queries < (1ll << 31),
                 "bad prompt score geometry");
+  WNW_CHECK_ARG(n_kv_heads >= 1 && n_heads >= 1 && n_heads % n_kv_heads == 0 && n_heads <= 65536,
+                "bad head counts %lld / %lld", (long long)n_heads, (long long)n_kv_heads);
+  const int64_t group = n_heads / n_kv_heads;
   if (batch == 0 || items == 0 || seq == 0 || max_audio == 0) return WNW_OK;
   WNW_CHECK_ARG(q && k && strides && audio_starts && audio_ends && workspace && (n_a == 0 || (a_heads && out_a)) &&
                     (n_kv == 0 || (kv_heads && out_h)),
@@ -626,7 +630,15 @@ extern "C" int wnw_prefill_scores(const void* q, const void* k, const void* mask
   WNW_CHECK_ARG(mask_dtype == WNW_F32 || mask_dtype == WNW_F16 || mask_dtype == WNW_BF16, "bad mask dtype %d",
                 mask_dtype);
   const int64_t per = 16 / elem_bytes(dtype);
-  for (int i = 0; i < 6; ++i) WNW_CHECK_ARG(strides[i] % per == 0, "q and k strides must be multiples of 16 bytes");
+  for (int i = 0; i < 6; ++i)
+    WNW_CHECK_ARG(strides[i] >= 0 && strides[i] % per == 0, "q and k strides must be multiples of 16 bytes");
+  WNW_CHECK_ARG(!mask || (strides[6] >= 0 && strides[7] >= 0), "negative mask stride");
+  for (int64_t i = 0; i < n_a; ++i)
+    WNW_CHECK_ARG(a_heads[i] >= 0 && a_heads[i] < n_heads, "class-A head %d is not one of %lld", a_heads[i],
+                  (long long)n_heads);
+  for (int64_t i = 0; i < n_kv; ++i)
+    WNW_CHECK_ARG(kv_heads[i] >= 0 && kv_heads[i] < n_kv_heads, "KV head %d is not one of %lld", kv_heads[i],
+                  (long long)n_kv_heads);
   WNW_CHECK_ARG(((uintptr_t)q % 16) == 0 && ((uintptr_t)k % 16) == 0, "q and k must be 16-byte aligned");
   WNW_CHECK_ARG(workspace_bytes >= wnw_prefill_scores_workspace_bytes(batch, items, seq, head_dim, max_queries, dtype),
                 "workspace too small");

@@ -98,10 +98,10 @@ def token_scores(q: Tensor, k: Tensor, attention_mask: Tensor | None, audio_star
         need = int(_lib.lib().wnw_prefill_scores_workspace_bytes(B, items, S, D, most, dt))
         ws = torch.empty(need, dtype=torch.uint8, device=dev)
         _lib.check(_lib.lib().wnw_prefill_scores(
-            _lib.ptr(q), _lib.ptr(k), _lib.ptr(m), strides, B, group, S, D, i32(audio_starts), i32(audio_ends),
-            i32(class_a_heads), len(class_a_heads), i32(kv_heads), len(kv_heads), 1 if last else 0, float(scaling), dt,
-            dt if m is None else _lib.dtype_code(m.dtype), width, most, _lib.ptr(out_a), _lib.ptr(out_h), _lib.ptr(ws),
-            need, _lib.stream_of(dev)), "prefill_scores")
+            _lib.ptr(q), _lib.ptr(k), _lib.ptr(m), strides, B, q.shape[1], k.shape[1], S, D, i32(audio_starts),
+            i32(audio_ends), i32(class_a_heads), len(class_a_heads), i32(kv_heads), len(kv_heads), 1 if last else 0,
+            float(scaling), dt, dt if m is None else _lib.dtype_code(m.dtype), width, most, _lib.ptr(out_a),
+            _lib.ptr(out_h), _lib.ptr(ws), need, _lib.stream_of(dev)), "prefill_scores")
     n = [e - a for a, e in zip(audio_starts, audio_ends)]
     return ([out_a[b, :n[b]] if class_a_heads else None for b in range(B)],
             [[out_h[b, i, :n[b]] for i in range(len(kv_heads))] for b in range(B)])
