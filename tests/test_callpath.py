@@ -1,8 +1,11 @@
 """The operators' native plain form (_callpath): the same results as the
 general path, and every call it does not take left to that path."""
+import sys
+
 import pytest
 import torch
 
+import wnw_amd
 from wnw_amd import _lib
 from wnw_amd.kv.fused_attn import AttnWorkspace, decode_attn
 from wnw_amd.wnw.kernels import fused_score_accumulate
@@ -19,6 +22,14 @@ def test_host_tensors_are_left_to_the_general_path():
         native.attn(q)
     with pytest.raises(_lib.WnwError, match="GPU tensors"):
         decode_attn(q, k, k, cu, 1.0)
+
+
+def test_missing_extension_names_the_build(monkeypatch):
+    monkeypatch.setattr(_lib, "_callpath", None)
+    monkeypatch.setitem(sys.modules, "wnw_amd._callpath", None)
+    monkeypatch.delattr(wnw_amd, "_callpath", raising=False)
+    with pytest.raises(RuntimeError, match="_callpath.so.*build the HIP extension"):
+        decode_attn(torch.zeros(2, 4, 128), torch.zeros(8, 128), torch.zeros(8, 128), torch.zeros(3), 1.0)
 
 
 def _segments(gpu, dtype, group, append):

@@ -11,6 +11,7 @@ import os
 
 import torch  # loads torch's HIP runtime first; the library binds to it
 
+_BUILD = "build the HIP extension first (python -c 'import __graft_entry__ as g; g.build()')"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libwnw_amd.so")
 
 WNW_OK, WNW_EINVAL, WNW_EHIP, WNW_ENOTSUP = 0, 1, 2, 3
@@ -108,9 +109,7 @@ def lib() -> ctypes.CDLL:
     global _lib
     if _lib is None:
         if not os.path.exists(LIB_PATH):
-            raise RuntimeError(
-                f"{LIB_PATH} is missing: build the HIP extension first "
-                "(python -c 'import __graft_entry__ as g; g.build()')")
+            raise RuntimeError(f"{LIB_PATH} is missing: {_BUILD}")
         handle = ctypes.CDLL(LIB_PATH)
         for name, (res, args) in _SIGNATURES.items():
             fn = getattr(handle, name)
@@ -125,11 +124,14 @@ _callpath = None
 
 def callpath():
     """The native form of the operators' plain calls (``_callpath.so``, built
-    with the library; raises if it has not been)."""
+    with the library against the installed torch; raises if it has not been)."""
     global _callpath
     if _callpath is None:
         lib()
-        from . import _callpath as mod
+        try:
+            from . import _callpath as mod
+        except ImportError as e:
+            raise RuntimeError(f"wnw_amd/_callpath.so is missing or does not load ({e}): {_BUILD}") from e
         from .kv.fused_attn import call_workspace
         from .wnw.kernels import call_score_workspace
 
