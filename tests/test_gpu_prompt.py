@@ -189,6 +189,31 @@ def test_token_scores(gpu, dtype, D, G, H, S, mode, mask):
                 torch.testing.assert_close(x.double(), y, atol=1e-6, rtol=1e-4)
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("deviation", [1.0, 3.0])
+def test_fp32_token_scores_no_less_exact_than_torch(gpu, monkeypatch, D, deviation):
+    """fp32 scores against 64 bits, beside the PyTorch form's, root mean square
+    over 16 inputs: 0.5 to 0.95 of it by the order of the sums; a dot as one
+    chain of multiply-adds is at 1.5 to 3."""
+    H, G, S = 3, 4, 900
+    cache = _Cache(_Config([0, 2], G, "last"), [14], [850])
+    native, sums = session.token_scores, {}
+    for seed in range(16):
+        q, k, _ = _qkv(gpu, 1, H * G, S, D, torch.float32, seed, "heads")
+        q, k = q * deviation, k[:, :H].contiguous()
+        want = _scores64(q.double(), k.double(), None, cache, H, G, D ** -0.5)
+        for name, f in (("kernel", native), ("torch", lambda *a: None)):
+            monkeypatch.setattr(session, "token_scores", f)
+            got = session.compute_prefill_scores(q, k, None, cache, 0, H, G, D ** -0.5)
+            for part, x, y in (("class A", got[0][0], want[0][0]), ("head", got[1][0][1], want[1][0][1])):
+                e = float((x.double() - y).norm() / y.norm())
+                sums[name, part] = sums.get((name, part), 0.0) + e * e
+    for part in ("class A", "head"):
+        ours, theirs = (sums[n, part] ** 0.5 / 4 for n in ("kernel", "torch"))
+        print(f"prompt scores D={D} deviation={deviation} {part}: {ours:.3e}, torch {theirs:.3e}", flush=True)
+        assert ours <= 1.2 * theirs, (part, ours, theirs)
+
+
 def _scores64(q, k, m, cache, H, G, scale):
     """compute_prefill_scores in 64 bits."""
     B, _, S, _ = q.shape

@@ -10,7 +10,7 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "wnw_common.h"
+#include "wnw_dot.h"
 
 namespace wnw {
 
@@ -24,10 +24,6 @@ struct PromptOps<bf16_t> {
   typedef __bf16 v4 __attribute__((ext_vector_type(4)));
   __device__ static f32x16 mma32(const u32x4& a, const u32x4& b, const f32x16& c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
-                                                   0, 0);
-  }
-  __device__ static f32x4 mma16(const u32x4& a, const u32x4& b, const f32x4& c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
                                                    0, 0);
   }
   __device__ static uint64_t read_tr(const uint8_t* lds) {
@@ -48,26 +44,12 @@ struct PromptOps<f16_t> {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
                                                   0);
   }
-  __device__ static f32x4 mma16(const u32x4& a, const u32x4& b, const f32x4& c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
-                                                  0);
-  }
   __device__ static uint64_t read_tr(const uint8_t* lds) {
     return __builtin_bit_cast(uint64_t,
                               __builtin_amdgcn_ds_read_tr16_b64_v4f16((__attribute__((address_space(3))) h4*)lds));
   }
   __device__ static uint32_t pack2(float a, float b) { return f32_to_f16_bits(a) | (f32_to_f16_bits(b) << 16); }
 };
-template <>
-struct PromptOps<float> {
-  __device__ static f32x4 mma16(const u32x4& a, const u32x4& b, f32x4 c) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[j]), __uint_as_float(b[j]), c, 0, 0, 0);
-    return c;
-  }
-};
-
 // ---------------------------------------------------------------------------
 // causal attention of a prompt (bf16 / f16, head_dim 64 or 128)
 // ---------------------------------------------------------------------------
@@ -317,8 +299,12 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PromptAttnParams p
 // keys as matrix operands) and streams the queries past them, 16 per matrix
 // tile, so K is read once per launch.  Latency bound (a few MB): the torch form
 // it replaces was ~10 launches per KV head plus an S x S mask, ~500 us a layer
-// at 4,564 rows of 8 KV heads (50 text rows); now 13.5 + 15.3 us.  Logits are 32-bit sums of exact 16-bit products
-// (that form rounded them to 16 bits twice).
+// at 4,564 rows of 8 KV heads (50 text rows); now 13.5 + 15.3 us.  Logits are
+// 32-bit sums of exact 16-bit products (that form rounded them to 16 bits twice);
+// fp32 dots are added as trees of chains of 8, no less exact than that form's
+// library products (as one chain 2-3 times their error for the last row; 4,564
+// rows 56 -> 67 us with the torch calls around the launches, 300 text rows of
+// 28 heads of 64 380 -> 520 us).
 static constexpr int kPsThreads = 256;
 static constexpr int kPsMax = 64;       // KV heads, class-A heads and samples a launch describes
 static constexpr int kPsQueries = 512;  // queries whose statistics sit in LDS at a time
@@ -354,7 +340,6 @@ __device__ __forceinline__ float mask_at(const void* m, int64_t i, int dtype) {
 template <typename T, int D, bool SUM>
 __global__ __launch_bounds__(kPsThreads) void prompt_score_kernel(PromptScoreParams p) {
   using Ge = PromptScoreGeom<T, D>;
-  using Ops = PromptOps<T>;
   constexpr int NC = Ge::NC, KT = Ge::KT, EPC = 16 / (int)sizeof(T);
   constexpr float kLowest = -3.402823466e38f;
   __shared__ float st[SUM ? 1 : 4][kPsQueries][2];
@@ -432,10 +417,7 @@ __global__ __launch_bounds__(kPsThreads) void prompt_score_kernel(PromptScorePar
       f32x4 v[KT];
 #pragma unroll
       for (int t = 0; t < KT; ++t) {
-        v[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int n = 0; n < NC; ++n) v[t] = Ops::mma16(kr[t][n], qc[n], v[t]);
-        v[t] *= p.scale;
+        v[t] = dot_rows<T, NC, sizeof(T) == 4 ? 2 : NC>(kr[t], qc) * p.scale;
       }
       if (p.mask) {  // wave-uniform, as the tests below
 #pragma unroll
