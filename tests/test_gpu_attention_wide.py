@@ -58,7 +58,7 @@ def test_many_segments_per_wave(gpu, dtype, G, D):
 
 @pytest.mark.parametrize("dtype,G,D", [("bfloat16", 4, 128), ("float16", 16, 128), ("bfloat16", 7, 64),
                                        ("float32", 2, 128)])
-@pytest.mark.parametrize("n_wg", [97, 256, 1100])
+@pytest.mark.parametrize("n_wg", [97, 150, 256, 1100])
 def test_two_level_merge(gpu, dtype, G, D, n_wg):
     """Segments of more than 32 pieces (merged block by block) side by side,
     with one-row and empty segments between, at piece counts around whole

@@ -12,9 +12,18 @@ static constexpr int kSplitWaves = 4;   // waves a workgroup's row range is cut 
 static constexpr int kPrevLogits = 16;  // pairs per sample the deferred form takes (<= 8 KV heads)
 static constexpr float kLog2e = 1.4426950408889634f;
 
+static constexpr int kMaxWgs = 2048;  // workgroups per launch at most
+
+// Two-level merge of long segments (streaming kernel): block partials, two per
+// 16 workgroups, and an arrival counter each.  They lie just before the
+// partials and counters of the segments, at distances that depend on G and D
+// alone, so a kernel finds them without arguments of their own.
 static constexpr int kPiecesPerBlock = 16;
-// Block partials of a launch of n_wg workgroups (two per 16 workgroups).
-constexpr int64_t attn_blocks(int64_t n_wg) { return 2 * (n_wg / kPiecesPerBlock + 1); }
+static constexpr int kMaxBlocks = 2 * (kMaxWgs / kPiecesPerBlock + 1);
+__host__ __device__ constexpr int64_t up256(int64_t x) { return (x + 255) / 256 * 256; }
+__host__ __device__ constexpr int64_t blk_counter_bytes() { return up256(kMaxBlocks * 4); }
+__host__ __device__ constexpr int64_t blk_ml_bytes(int64_t G) { return up256(kMaxBlocks * G * 2 * 4); }
+__host__ __device__ constexpr int64_t blk_acc_bytes(int64_t GD) { return up256(kMaxBlocks * GD * 4); }
 
 struct AttnParams {
   const void* q;        // [n_seg, G, D]
@@ -66,12 +75,6 @@ struct AttnParams {
   int64_t pv_acc_len;
   int32_t pv_nblk;  // 256-token blocks per sample
   int32_t pv_slices;  // samples x pv_nblk (<= the grid)
-  // two-level merge of long segments (streaming kernel, BLK instances; last, so that the
-  // fields every launch reads keep their cache lines): block partials and
-  // their arrival counters, attn_blocks(grid) of each
-  float* blk_acc;
-  float* blk_ml;
-  int32_t* blk_counters;
 };
 
 // Launches kernel WNW_ATTN_{MFMA,VALU,STREAM} for element type T.

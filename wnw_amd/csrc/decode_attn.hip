@@ -30,40 +30,33 @@ static DeviceInfo& device_info() {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
       cus = 256;
     di.cus = cus;
-    di.max_wg = cus * 8;
+    di.max_wg = std::min(cus * 8, kMaxWgs);
   }
   return di;
 }
 
 struct WsLayout {
   int64_t counters, ml, acc, total;
-  int64_t blk_counters, blk_ml, blk_acc;
-  int64_t slots;
 };
+static int64_t blk_bytes(int64_t G, int64_t D) { return blk_counter_bytes() + blk_ml_bytes(G) + blk_acc_bytes(G * D); }
 
-// Arrival counters of cap_seg segments and `blocks` block partials first
-// (their place depends on cap_seg alone: a launch with another group or
-// head_dim finds them cleared), then the (m, l) pairs and the accumulators of
-// `slots` partial slots and of the block partials.
-static WsLayout make_layout(int64_t cap_seg, int64_t slots, int64_t G, int64_t D, int64_t blocks) {
+// Arrival counters of the block partials and of cap_seg segments first (their
+// place depends on nothing but cap_seg: a launch with another group or
+// head_dim finds them cleared), then the (m, l) pairs and the accumulators,
+// each time the block partials' before those of `slots` partial slots.
+static WsLayout make_layout(int64_t cap_seg, int64_t slots, int64_t G, int64_t D) {
   WsLayout L;
-  L.slots = slots;
-  auto up = [](int64_t x) { return (x + 255) / 256 * 256; };
-  L.counters = 0;
-  L.blk_counters = cap_seg * 4;
-  L.ml = up((cap_seg + blocks) * 4);
-  L.acc = L.ml + up(L.slots * G * 2 * 4);
-  L.blk_ml = L.acc + up(L.slots * G * D * 4);
-  L.blk_acc = L.blk_ml + up(blocks * G * 2 * 4);
-  L.total = L.blk_acc + up(blocks * G * D * 4);
+  L.counters = blk_counter_bytes();
+  L.ml = L.counters + up256(cap_seg * 4) + blk_ml_bytes(G);
+  L.acc = L.ml + up256(slots * G * 2 * 4) + blk_acc_bytes(G * D);
+  L.total = L.acc + up256(slots * G * D * 4);
   return L;
 }
 
 // Caller-owned workspace: sized before the grid is known, so for the
 // largest grid a launch may use.
 static WsLayout ws_layout(int64_t n_seg, int64_t G, int64_t D) {
-  const int64_t wg = device_info().max_wg;
-  return make_layout(n_seg, wg + n_seg, G, D, attn_blocks(wg));
+  return make_layout(n_seg, device_info().max_wg + n_seg, G, D);
 }
 
 // ---------------------------------------------------------------------------
@@ -78,12 +71,10 @@ static WsLayout ws_layout(int64_t n_seg, int64_t G, int64_t D) {
 // launch leaves the counters of its segments at zero, the others are never
 // touched, and the array is zero at load (cleared again on first use).
 // WNW_NOALLOC_SCRATCH_BYTES bound a call's partials and segment counters; the
-// block partials (grids of up to kNoAllocWgs, two workgroups per CU) have
-// room of their own.
+// block partials have room of their own (grids of up to kNoAllocWgs).
 static constexpr int64_t kNoAllocWgs = 1024;
-static constexpr int64_t kNoAllocBlocks = attn_blocks(kNoAllocWgs);
 static constexpr int64_t kNoAllocBytes =
-    WNW_NOALLOC_SCRATCH_BYTES + kNoAllocBlocks * (4 + kMaxGroup * (256 + 2) * 4) + 4 * 256;
+    WNW_NOALLOC_SCRATCH_BYTES + blk_counter_bytes() + blk_ml_bytes(kMaxGroup) + blk_acc_bytes(kMaxGroup * 256);
 static __device__ __align__(256) uint8_t g_attn_scratch[kNoAllocBytes];
 
 struct ScratchSlot {
@@ -136,7 +127,7 @@ static int noalloc_scratch(hipStream_t st, void** out) {
     sl.ptr = p;
   }
   if (!sl.cleared) {
-    const int64_t n = (int64_t)WNW_NOALLOC_MAX_SEG + kNoAllocBlocks;  // counters, 4 bytes each
+    const int64_t n = (int64_t)WNW_NOALLOC_MAX_SEG + blk_counter_bytes() / 4;  // counters, 4 bytes each
     hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (uint32_t*)sl.ptr, n);
     WNW_CHECK_HIP(hipGetLastError(), "clearing the attention scratch counters");
     sl.cleared = true;
@@ -206,12 +197,12 @@ int decode_attn_impl(const void* q, const void* k, const void* v, const int32_t*
     const bool narrow = dtype != WNW_F32 && head_dim <= 128 && group <= kMaxGroupS;
     const int64_t P_lim = std::min<int64_t>((int64_t)di.cus * (narrow ? 1 : 2), std::max<int64_t>(1, (total_rows + 63) / 64));
     P = std::min(P, kNoAllocWgs);
-    const WsLayout lim = make_layout(WNW_NOALLOC_MAX_SEG, std::max(P, P_lim) + n_seg, group, head_dim, 0);
-    WNW_CHECK_ARG(lim.total <= WNW_NOALLOC_SCRATCH_BYTES,
+    L = make_layout(WNW_NOALLOC_MAX_SEG, std::max(P, P_lim) + n_seg, group, head_dim);
+    const int64_t need = L.total - blk_bytes(group, head_dim);
+    WNW_CHECK_ARG(need <= WNW_NOALLOC_SCRATCH_BYTES,
                   "this launch needs %lld bytes of split-K scratch; the no-alloc entry point holds %lld "
                   "(fewer segments or a smaller group / head_dim fit)",
-                  (long long)lim.total, (long long)WNW_NOALLOC_SCRATCH_BYTES);
-    L = make_layout(WNW_NOALLOC_MAX_SEG, std::max(P, P_lim) + n_seg, group, head_dim, kNoAllocBlocks);
+                  (long long)need, (long long)WNW_NOALLOC_SCRATCH_BYTES);
     const int rc = noalloc_scratch((hipStream_t)stream, &workspace);
     if (rc != WNW_OK) return rc;
   } else {
@@ -231,9 +222,6 @@ int decode_attn_impl(const void* q, const void* k, const void* v, const int32_t*
   ap.lse = lse;
   ap.part_ml = (float*)((char*)workspace + L.ml);
   ap.part_acc = (float*)((char*)workspace + L.acc);
-  ap.blk_counters = (int32_t*)((char*)workspace + L.blk_counters);
-  ap.blk_ml = (float*)((char*)workspace + L.blk_ml);
-  ap.blk_acc = (float*)((char*)workspace + L.blk_acc);
   ap.err = device_error_word();
   ap.split_inv = ~0ull / (uint64_t)(P * kSplitWaves) + 1;  // ceil(2^64 / (P * kSplitWaves))
   ap.phys_rows = kv_rows;

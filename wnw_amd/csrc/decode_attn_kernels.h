@@ -541,10 +541,29 @@ __device__ __forceinline__ void wait_vmcnt() {
 // 16; and of two segments with a block start in one bucket the earlier one's
 // is not its first block (it has more than 32 pieces, the later segment
 // starts where it ends or after) and the later one's is its first.
+// In a launch of fewer than kBlkWgsFull workgroups the blocks end at about the
+// same time, and it takes a third round trip to lose: 133 workgroups, 43-44
+// pieces 12.1 -> 13.0 us by blocks, 66 pieces 14.5 -> 11.6.
 static constexpr int kBlk = 16;
 static constexpr int kBlkMin = 32;
+static constexpr int kBlkMinSmall = 48;
+static constexpr int kBlkWgsFull = 192;
+__device__ __forceinline__ int blk_min(int wgs) { return wgs < kBlkWgsFull ? kBlkMinSmall : kBlkMin; }
 static_assert(kBlk == kPiecesPerBlock, "the workspace is sized for this block");
 __device__ __forceinline__ int block_index(int bucket, int j) { return 2 * (bucket + j) + (j > 0 ? 1 : 0); }
+
+// The block partials and their counters, found from the segments' ones: as
+// three more arguments they cost a kernel that has no scalar register left up
+// to 0.5 us a launch, also where no segment has more than kBlkMin pieces.
+struct BlkArgs {
+  float* acc;
+  float* ml;
+  int32_t* counters;
+};
+__device__ __forceinline__ BlkArgs blk_args(const AttnParams& p, int GD) {
+  return BlkArgs{p.part_acc - blk_acc_bytes(GD) / 4, p.part_ml - blk_ml_bytes(p.G) / 4,
+                 p.counters - blk_counter_bytes() / 4};
+}
 
 // Merge of np partials of segment s (slots s0 .. s0 + np - 1) by threads
 // t = 0 .. nt - 1: into the output, or (BLK, with dst_acc) as one partial there.
@@ -558,7 +577,7 @@ __device__ __forceinline__ int block_index(int bucket, int j) { return 2 * (buck
 // a segment's block partials (block_index), the first at index s0.
 template <typename T, bool BLK>
 __device__ __forceinline__ void combine_pieces(const AttnParams& p, int D, int64_t s0, int np, int64_t s, int t,
-                                               int nt, bool blocks = false, float* dst_acc = nullptr,
+                                               int nt, const BlkArgs* blocks = nullptr, float* dst_acc = nullptr,
                                                float* dst_ml = nullptr) {
   // wave-uniform values: scalar, so the buffer descriptors below live in SGPRs
   s0 = uni(s0);
@@ -573,9 +592,9 @@ __device__ __forceinline__ void combine_pieces(const AttnParams& p, int D, int64
   const int GD4 = GD / 4;
   const int span = BLK && blocks ? 2 * np : np;
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
-      (BLK && blocks ? p.blk_acc : p.part_acc) + s0 * GD, 0, span * GD * 4, kRsrc3);
+      (BLK && blocks ? blocks->acc : p.part_acc) + s0 * GD, 0, span * GD * 4, kRsrc3);
   const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(
-      (BLK && blocks ? p.blk_ml : p.part_ml) + s0 * G * 2, 0, span * G * 8, kRsrc3);
+      (BLK && blocks ? blocks->ml : p.part_ml) + s0 * G * 2, 0, span * G * 8, kRsrc3);
   for (int i4 = t; i4 < GD4; i4 += nt) {
     const int g = (4 * i4) / D;
     float M = kNegBig, L = 0.f;
@@ -1211,8 +1230,8 @@ struct SStep {
 // table and fused append only), an instance of its own so that the other
 // launches carry none of its code or argument loads.
 // BLK: merge segments of more than kBlkMin pieces in two levels, an instance of
-// its own because that code costs every launch that never takes it ~0.25 us
-// (20.15 -> 20.4 us per fused launch at 64 segments of up to 7,564 rows).
+// its own because that code, though out of the way, costs a launch that never
+// takes it up to 0.3 us by the registers the compiler gives it.
 template <typename T, int D, int NW, int QD, bool XL, bool APPEND, bool DIRECT, bool PV, bool BLK>
 // The fields read first lead the argument list as scalars: the build asks
 // for 16 preloaded argument dwords (-amdgpu-kernarg-preload-count), of which
@@ -2031,10 +2050,10 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
     if (ps >= 0) {
       int32_t last = pn;
       WNW_GLOBAL int32_t* c = gptr_w<int32_t>(p.counters) + ps;
-      if (BLK && pn >= kBlkMin) {
+      if (BLK && __builtin_expect(pn >= blk_min(sl.P), 0)) {
         const int32_t j = ((int32_t)blockIdx.x - pf) / kBlk;
         last = min(kBlk - 1, pn - kBlk * j);
-        c = gptr_w<int32_t>(p.blk_counters) + block_index(pf / kBlk, j);
+        c = gptr_w<int32_t>(blk_args(p, GD).counters) + block_index(pf / kBlk, j);
       }
       f = __hip_atomic_fetch_add(c, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == last;
     }
@@ -2062,18 +2081,25 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
     const bool k = both ? tid >= NT / 2 : last == 2;  // uniform per wave
     const int t = both && k ? tid - NT / 2 : tid;
     const int32_t ps = k ? ps1 : ps0, np = (k ? pn1 : pn0) + 1, pf = (int32_t)(k ? pf1 : pf0);
-    const bool blk = BLK && np > kBlkMin;
-    const int32_t j = blk ? ((int32_t)blockIdx.x - pf) / kBlk : 0;
-    const int32_t bi = blk ? block_index(pf / kBlk, j) : 0;
-    const int64_t slot = (int64_t)pf + kBlk * j + ps;
-    combine_pieces<T, BLK>(p, D, slot, blk ? min(kBlk, np - kBlk * j) : np, ps, t, nt, false,
-                           blk ? p.blk_acc + (int64_t)bi * GD : nullptr, BLK ? p.blk_ml + (int64_t)bi * G * 2 : nullptr);
-    if (t == 0)
-      __hip_atomic_store(BLK && blk ? gptr_w<int32_t>(p.blk_counters) + bi : gptr_w<int32_t>(p.counters) + ps, 0,
-                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // the segments' block arrivals, and the merge of the blocks by the last
-    const int at = BLK ? last & ((pn0 >= kBlkMin ? 1 : 0) | (pn1 >= kBlkMin ? 2 : 0)) : 0;  // workgroup-uniform
-    if (BLK && at) {
+    // bit i: segment i merges block by block (workgroup-uniform)
+    const int bm = BLK ? blk_min(uni(sl.P)) : 0;
+    const int at = BLK ? last & ((pn0 >= bm ? 1 : 0) | (pn1 >= bm ? 2 : 0)) : 0;
+    if (__builtin_expect(at == 0, 1)) {
+      combine_pieces<T, false>(p, D, (int64_t)pf + ps, np, ps, t, nt);
+      if (t == 0)
+        __hip_atomic_store(gptr_w<int32_t>(p.counters) + ps, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else if constexpr (BLK) {
+      const BlkArgs ba = blk_args(p, GD);
+      const bool blk = np > bm;
+      const int32_t j = blk ? ((int32_t)blockIdx.x - pf) / kBlk : 0;
+      const int32_t bi = blk ? block_index(pf / kBlk, j) : 0;
+      const int64_t slot = (int64_t)pf + kBlk * j + ps;
+      combine_pieces<T, true>(p, D, slot, blk ? min(kBlk, np - kBlk * j) : np, ps, t, nt, nullptr,
+                              blk ? ba.acc + (int64_t)bi * GD : nullptr, ba.ml + (int64_t)bi * G * 2);
+      if (t == 0)
+        __hip_atomic_store(blk ? gptr_w<int32_t>(ba.counters) + bi : gptr_w<int32_t>(p.counters) + ps, 0,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      // the segments' block arrivals, and the merge of the blocks by the last
       wait_vmem();
       __syncthreads();  // block partials complete, is_last read by everyone
       if (tid < 2) {
@@ -2089,7 +2115,7 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
       for (int i = 0; i < 2; ++i) {
         if (!((last2 >> i) & 1)) continue;  // workgroup-uniform
         const int32_t s2 = i ? ps1 : ps0, b0 = block_index((int32_t)(i ? pf1 : pf0) / kBlk, 0);
-        combine_pieces<T, BLK>(p, D, b0, (i ? pn1 : pn0) / kBlk + 1, s2, tid, NT, true);
+        combine_pieces<T, true>(p, D, b0, (i ? pn1 : pn0) / kBlk + 1, s2, tid, NT, &ba);
         if (tid == 0)
           __hip_atomic_store(gptr_w<int32_t>(p.counters) + s2, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
@@ -2281,10 +2307,11 @@ static hipError_t launch_stream_k(const AttnParams& ap, int64_t n_wg, hipStream_
 // kBlkWgs workgroups, eight or more of them per segment, may well hold segments of
 // more than kBlkMin pieces and takes the instance that merges those in two
 // levels: 8 segments, two of 22,628 rows (95 pieces each) 24.9 -> 20.2 us; 16
-// segments, fp16, 16 heads, up to 86 pieces 32.4 -> 26.9 us.  With more segments or
-// fewer workgroups the long ones rarely pass 32 pieces and the instance's
-// cost is not earned (64 segments, 16 of ~7,300 ragged rows: 31.5 -> 32.2 us; 41
-// workgroups, 8 segments: 10.0 -> 10.4 us).  With q in registers there is
+// segments, fp16, 16 heads, up to 86 pieces 32.4 -> 26.9 us.  The host knows the
+// rows in all and not the longest segment: of 174 launches of 1 to 32 segments
+// of 8,500 to 100,000 rows the 125 with longer ones gain 4 % (33-48 pieces), 20 %
+// (up to 80) and 86 % (more) on average, the others lose 2 % to this instance.
+// With more segments or fewer workgroups the long ones rarely pass 32 pieces.  With q in registers there is
 // the one direct instance (such launches' accumulators are wide and the
 // chain of round trips long).
 static constexpr int kBlkWgs = 128;
