@@ -549,12 +549,27 @@ def test_fused_append_pieces_of_whole_steps(gpu, case):
         _check_append(_append_case(gpu, lens, 4, 128, dtype, seed=len(lens)), dtype)
 
 
-@pytest.mark.parametrize("dtype,G,D", [("float32", 4, 128), ("bfloat16", 16, 128), ("bfloat16", 4, 256)])
+@pytest.mark.parametrize("dtype,G,D", [("float32", 4, 128), ("bfloat16", 16, 128), ("bfloat16", 4, 256),
+                                       ("float32", 4, 256), ("float32", 16, 256)])
 def test_fused_append_other_kernels(gpu, dtype, G, D):
-    """Where the streaming kernel does not apply (fp32, group > 8, head_dim
-    256) the entry point runs the in-place append, then the attention."""
+    """The forms outside 16-bit rows of up to 256 bytes and groups of up to 8:
+    the streaming kernel's with q in registers (the first three), and fp32
+    head_dim 256, whose rows it does not take: there the entry point runs the
+    in-place append, then the attention (the VALU kernel)."""
     lens = [0, 3, 700, 129, 1, 2000, 45]
     _check_append(_append_case(gpu, lens, G, D, dtype, seed=3), dtype)
+
+
+@pytest.mark.parametrize("G", [4, 16])
+def test_fused_append_with_scores_fp32_256(gpu, G):
+    """fp32 head_dim 256: the VALU kernel keeps no logits, so the scoring pass
+    reads K again (attn_score_kernel) after the append and the attention."""
+    lens = [40, 300, 17, 1000, 64, 2, 513, 90]
+    r = _append_case(gpu, lens, G, 256, "float32", seed=4, score=(4, [0, 1, 0, 1], [3, 0], [17, 2]))
+    _check_append(r, "float32")
+    acc, ref_acc = r["extra"]
+    ok, msg = allclose_report(acc.cpu().numpy().astype(np.float64), ref_acc, 1e-6, 1e-3)
+    assert ok, msg
 
 
 def test_fused_append_capacity_is_refused(gpu):

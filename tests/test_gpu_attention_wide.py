@@ -10,6 +10,7 @@ import pytest
 
 from tests.helpers import allclose_report
 from tests.test_gpu_attention import _append_case, _check_append, _run_case, _tol
+from wnw_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -45,6 +46,13 @@ def test_append_with_scores(gpu, dtype, G, D):
     acc, ref = r["extra"]
     ok, msg = allclose_report(acc.cpu().numpy().astype(np.float64), ref, 1e-6, 1e-3)
     assert ok, msg
+
+
+@pytest.mark.parametrize("dtype,G,D", [("float32", 4, 128), ("bfloat16", 16, 128), ("bfloat16", 4, 256)])
+def test_capacity_is_refused(gpu, dtype, G, D):
+    """A segment without room for its new row: WNW_DEVERR_CAPACITY, and the
+    row is not stored."""
+    _check_append(_append_case(gpu, [40, 300, 5, 77], G, D, dtype, seed=9, short_cap=1), dtype, err=_lib.DEVERR_CAPACITY)
 
 
 @pytest.mark.parametrize("dtype,G,D", [("float32", 4, 128), ("bfloat16", 16, 128), ("bfloat16", 5, 256)])

@@ -5,6 +5,8 @@ Attention: 16-bit outputs and 16-bit weights in the value product, relative
 2-norm error of at most 4e-3 (bf16, 2^-8 steps) / 5e-4 (f16).  Scores: 32-bit
 logits of exact 16-bit products, 32-bit sums: 1e-6 + 1e-4 |ref| (weights in
 [0, 1], the exponential's argument error scales with the logits)."""
+import ctypes
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -25,7 +27,8 @@ def _qkv(dev, B, H, S, D, dtype, seed, layout):
 
 
 @pytest.mark.parametrize("S", [1, 2, 31, 32, 33, 63, 64, 65, 127, 128, 129, 193, 500])
-@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.float16, 128), (torch.bfloat16, 64)])
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.float16, 128), (torch.bfloat16, 64),
+                                     (torch.float16, 64)])
 @pytest.mark.parametrize("layout", ["heads", "rows"])
 def test_causal_attention(gpu, S, dtype, D, layout):
     q, k, v = _qkv(gpu, 2, 3, S, D, dtype, S, layout)
@@ -35,6 +38,26 @@ def test_causal_attention(gpu, S, dtype, D, layout):
     s = (q.double() @ k.double().transpose(-1, -2).contiguous()) * 0.11
     s = s + torch.full((S, S), float("-inf"), device=gpu, dtype=torch.float64).triu_(1)
     ref = s.softmax(-1) @ v.double().contiguous()
+    err = float((out.double() - ref).norm() / ref.norm())
+    assert err < (4e-3 if dtype == torch.bfloat16 else 5e-4), err
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.float16, 64)])
+@pytest.mark.parametrize("H,Hkv", [(8, 2), (7, 1)])
+def test_causal_attention_grouped(gpu, dtype, D, H, Hkv):
+    """The C entry point with fewer KV heads than query heads."""
+    B, S, scale = 2, 150, 0.1
+    q = _qkv(gpu, B, H, S, D, dtype, 1, "rows")[0]
+    k, v, _ = _qkv(gpu, B, Hkv, S, D, dtype, 2, "heads")
+    out = torch.empty_like(q)
+    strides = (ctypes.c_int64 * 12)(*(t.stride(i) for t in (q, k, v, out) for i in range(3)))
+    _lib.check(_lib.lib().wnw_prefill_attn(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), B, H, Hkv, S, D, strides, scale,
+                                           _lib.dtype_code(dtype), _lib.ptr(out), _lib.stream_of(gpu)))
+    kk, vv = (t.repeat_interleave(H // Hkv, dim=1) for t in (k, v))
+    assert torch.equal(out, prompt.causal_attention(q, kk, vv, scale))
+    s = (q.double() @ kk.double().transpose(-1, -2).contiguous()) * scale
+    s = s + torch.full((S, S), float("-inf"), device=gpu, dtype=torch.float64).triu_(1)
+    ref = s.softmax(-1) @ vv.double().contiguous()
     err = float((out.double() - ref).norm() / ref.norm())
     assert err < (4e-3 if dtype == torch.bfloat16 else 5e-4), err
 

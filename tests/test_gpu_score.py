@@ -251,7 +251,8 @@ def test_attn_score_many_samples(keep_logits):
 
 
 def test_fused_score_accumulate_many_samples():
-    """fused_score_accumulate with the long (16-iteration) scoring workgroups."""
+    """fused_score_accumulate over enough items for several per CU: 24 of them,
+    in 22 slices each."""
     dev = torch.device("cuda", 0)
     rng = np.random.default_rng(13)
     S, nh, D = 24, 2, 128
