@@ -204,9 +204,9 @@ int wnw_compact_segments(const void* src_k, const void* src_v, void* dst_k,
  * arrival counters; it must be cleared once with wnw_workspace_init before
  * its first use and may then be reused by any number of launches on one
  * stream (every launch leaves the counters at zero).  The counters occupy the
- * front, as many bytes as n_seg asks for, and the partials follow them, so a
- * launch with another n_seg turns partial bytes into counters and the
- * reverse: clear the workspace again whenever n_seg changes.
+ * front, a fixed part and as many bytes as n_seg asks for, and the partials
+ * follow them, so a launch with another n_seg turns partial bytes into counters
+ * and the reverse: clear the workspace again whenever n_seg changes.
  */
 int64_t wnw_decode_attn_workspace_bytes(int64_t n_seg, int64_t group,
                                         int64_t head_dim);
@@ -281,8 +281,9 @@ int wnw_decode_attn_ex(const void* q, const void* k, const void* v,
                        int64_t workspace_bytes, int kernel, int64_t n_wg,
                        void* stream);
 
-/* Limits of wnw_decode_attn_noalloc: the size of the library's own split-K
- * scratch on each device, and the segments its counters region holds. */
+/* Limits of wnw_decode_attn_noalloc: what the partial slots and segment
+ * counters of a call may take of the library's own split-K scratch on each
+ * device, and the segments its counters region holds. */
 #define WNW_NOALLOC_SCRATCH_BYTES (16ll << 20)
 #define WNW_NOALLOC_MAX_SEG 4096
 
@@ -292,11 +293,15 @@ int wnw_decode_attn_ex(const void* q, const void* k, const void* v,
  * reference; it is for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  The split-K partials and arrival counters live in a
- * file-scope device array of the library, WNW_NOALLOC_SCRATCH_BYTES per
- * device, held until the process ends.  Limits: n_seg <= WNW_NOALLOC_MAX_SEG,
- * and (grid + n_seg) partial slots of group * (head_dim + 2) floats must fit
- * the array (n_seg 512, group 4, head_dim 128 needs ~1.6 MB); a larger call
- * returns WNW_EINVAL with the bytes it would need.  Every call on a device
+ * file-scope device array of the library, held until the process ends:
+ * WNW_NOALLOC_SCRATCH_BYTES per device for the slots and counters of the
+ * segments, and ~4 MiB more for the block partials that long segments merge
+ * through, which no limit concerns.  Limits: n_seg <= WNW_NOALLOC_MAX_SEG, and
+ * (workgroups + n_seg) partial slots of group * (head_dim + 2) floats must fit
+ * the former, counting one workgroup per 64 rows, up to one per CU for 16-bit
+ * rows of up to 128 elements and groups of up to 8 and up to two per CU
+ * otherwise, whatever grid is launched (n_seg 512, group 4, head_dim 128 needs
+ * ~1.6 MB); a larger call returns WNW_EINVAL with the bytes it would need.  Every call on a device
  * shares that device's array, so calls that overlap on one device (other
  * streams, other threads) race: order them on one stream.  The first call on
  * a device clears the counters with a fill kernel on `stream`.

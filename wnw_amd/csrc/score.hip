@@ -19,10 +19,11 @@
 // accumulator once per token: no atomics, deterministic results.
 //
 // Row dot products are 16 x 16 matrix instructions (rows x heads) in the
-// fused_score_accumulate passes.  In attn_score_kernel (kept for callers
-// without room for the logits) a row of D elements is read by D / EPC lanes,
-// 16 bytes each, and reduced across those lanes with a butterfly; q lives in
-// LDS as fp32.
+// fused_score_accumulate passes.  In attn_score_kernel (where no logits were
+// kept: callers without room for them, fp32 head_dim 256, whose attention
+// kernel keeps none, more than 64 KV heads) a row of D elements is read by
+// D / EPC lanes, 16 bytes each, and reduced across those lanes with a
+// butterfly; q lives in LDS as fp32.
 #include <math.h>
 
 #include <algorithm>
@@ -336,8 +337,13 @@ __device__ __forceinline__ u32x4 load_chunk(const T* p, bool aligned) {
   return r;
 }
 
-// Slices per item: enough workgroups for two per CU of a 256-CU device, each
-// still with a few 16-row tiles (8 items of 7,564 rows: 64 slices of 118 rows).
+// Slices per item, from the number of items alone (the workspace is sized
+// before the lengths are known): two workgroups per CU of a 256-CU device from
+// 4 items on (8 items of 7,564 rows: 64 slices of 118 rows), at most 128 slices,
+// which the merge takes two per lane, and at least 8.  One to three items thus
+// fill half to all of the CUs once, and the slices of short items hold less
+// than a tile (300 rows: 2-3 rows each; such a call is bound by its two
+// launches, 10.2 us like the 32 slices of the earlier kernels).
 static int64_t score_slices(int64_t n_samples) {
   return std::min<int64_t>(128, std::max<int64_t>(8, (512 + n_samples - 1) / std::max<int64_t>(n_samples, 1)));
 }
@@ -345,9 +351,10 @@ static int64_t score_slices(int64_t n_samples) {
 // Both passes, one workgroup per slice of an item's rows (SCORE 0: the
 // slice's partial softmax statistics of every head; SCORE 1: every head's
 // statistics merged, then each audio row's weights summed over the heads and
-// added to its accumulator entry).  The passes cut the rows alike, so the
-// second one's K comes from the L2 of the XCD that the first one's
-// workgroups filled.  Bound by the K stream and by two launches' fixed round
+// added to its accumulator entry).  The passes cut the rows alike, so as long
+// as K fits the eight L2s (4 MB each) the second one's comes from the L2 of the
+// XCD that the first one's workgroups filled; larger K (16 items of 24,000 bf16
+// rows: 98 MB) is streamed twice.  Bound by the K stream and by two launches' fixed round
 // trips; a row dot by 16-lane butterflies (six lane exchanges per row and
 // head) had bound it before: 25.1 + 10.4 us for 8 items of 7,564 rows, 4 heads,
 // bf16 D = 128 (15.5 MB), now 6.4 + 7.4 us.
