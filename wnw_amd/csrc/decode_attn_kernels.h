@@ -46,6 +46,7 @@
 #include <math.h>
 
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "decode_attn.h"
@@ -1029,7 +1030,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_mfma_kernel(AttnParams p) {
 // (MI355X, per launch): fp32 D = 128, G = 4, 5,632 rows 74.8 -> 14.2 us (the
 // VALU kernel read each lane's own row, 512 bytes apart, one step at a time;
 // the separate append launch of 4.8 us is gone too); bf16 D = 256, G = 4,
-// 35 MB 106.7 -> 27.0 us; fp16 D = 128, G = 16, 40 MB 43.0 -> 32.4 us (MFMA
+// 35 MB 106.7 -> 23.6 us; fp16 D = 128, G = 16, 40 MB 43.0 -> 32.4 us (MFMA
 // kernel: V transposed by 16-bit LDS reads).
 //
 // Each wave owns a contiguous quarter of its workgroup's row range and walks
@@ -1045,9 +1046,10 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_mfma_kernel(AttnParams p) {
 //       K operand read row by row from LDS (16-byte chunks XOR-swizzled by
 //       the row, so the 16 rows of one read hit distinct banks);
 //   (fp32: v_mfma_f32_16x16x4_f32, 32-bit operands and sums throughout;
-//   16-bit rows of 256: that instruction for O^T, weights kept in 32 bits and
-//   V widened, since a 16-bit pair drops f16 weights below 2^-25 of a wave's
-//   largest, and inf * (hi + lo) is NaN: 23.4 -> 27.0 us at 35 MB)
+//   16-bit rows of 256: weights of 32 bits for O^T, since a 16-bit pair drops
+//   f16 weights below 2^-25 of a wave's largest, and inf * (hi + lo) is NaN.
+//   f16: that instruction, V widened; bf16: three products with the weight's
+//   bits 8 at a time, exact; 23.4 -> 27.0 and 23.6 us at 36 MB)
 //   O^T += V^T x P^T: D/16 tiles of v_mfma_f32_16x16x16, two per tile (P
 //       split into hi + lo halves); the V^T operand comes from one
 //       ds_read_b64_tr_b16 per lane and tile (4 rows x 1 column each),
@@ -1299,7 +1301,10 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
   constexpr int kSaveRows = stream_save_rows(G_::RB);
   constexpr int kHeads = stream_heads(QD);
   constexpr bool kF32 = sizeof(T) == 4;
-  constexpr bool kP32 = kF32 || D > 128;  // 32-bit weights in the value product
+  // weights of 32 bits in the value product: as 32-bit operands, or (bf16) as
+  // three 16-bit ones
+  constexpr bool kP32 = kF32 || (D > 128 && !std::is_same<T, bf16_t>::value);
+  constexpr bool kP3 = D > 128 && std::is_same<T, bf16_t>::value;
   constexpr int NT = NW * 64;
   constexpr int RB = G_::RB, SB = G_::SB, NI = G_::NI, RPI = G_::RPI, CH = G_::CH, NC = G_::NC, NTD = G_::NTD;
   constexpr int QX = QD + (APPEND ? 1 : 0);  // first-step loads besides K and V: q (and the new row)
@@ -1689,8 +1694,29 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
     }
     // P = hi + lo, each a 16-bit float: PV runs as two MFMAs with ~16 (bf16) to
     // ~22 bits (f16, down to 2^-25 of the wave's maximum) of P
-    uint64_t ph = 0, pl = 0;
-    if constexpr (!kP32) {
+    uint64_t ph = 0, pm = 0, pl = 0;
+    if constexpr (kP3) {
+      // P = its bits 8 at a time, exactly; a part or a repeated row's weight
+      // that would be 0 is 2^-126 instead (see the 32-bit product below)
+      uint32_t hb[4], mb[4], lb[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t b = __float_as_uint(4 * lq + i < nvalid ? pv[i] : 0.f);
+        hb[i] = b & 0xffff0000u;
+        const float r = __uint_as_float(b) - __uint_as_float(hb[i]);
+        mb[i] = __float_as_uint(r) & 0xffff0000u;
+        lb[i] = __float_as_uint(r - __uint_as_float(mb[i]));
+        hb[i] = max(hb[i], 0x00800000u);
+        mb[i] = max(mb[i], 0x00800000u);
+        lb[i] = max(lb[i], 0x00800000u);
+      }
+      auto pack = [](const uint32_t* x) {
+        return (uint64_t)((x[0] >> 16) | (x[1] & 0xffff0000u)) | ((uint64_t)((x[2] >> 16) | (x[3] & 0xffff0000u)) << 32);
+      };
+      ph = pack(hb);
+      pm = pack(mb);
+      pl = pack(lb);
+    } else if constexpr (!kP32) {
       const uint32_t h01 = Ops::pack2(pv[0], pv[1]), h23 = Ops::pack2(pv[2], pv[3]);
       const uint32_t l01 = Ops::pack2(pv[0] - Ops::to_f32(h01 & 0xffffu), pv[1] - Ops::to_f32(h01 >> 16));
       const uint32_t l23 = Ops::pack2(pv[2] - Ops::to_f32(h23 & 0xffffu), pv[3] - Ops::to_f32(h23 >> 16));
@@ -1748,7 +1774,7 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
             acc[4 * u + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], w, acc[4 * u + j], 0, 0, 0);
         }
       }
-    } else {
+    } else if constexpr (!kF32) {
       const int r = 4 * lq + (lc >> 2);
       const int sw = 2 * (r & 3);
       const uint8_t* rowp = vbuf + r * RB + (lc & 1) * 8;
@@ -1757,6 +1783,7 @@ __global__ __launch_bounds__(NW * 64, D * sizeof(T) > 256 ? 1 : 2) void attn_str
         const int chunk = (2 * t + ((lc & 3) >> 1)) ^ sw;
         const uint64_t a = Ops::vt(rowp + chunk * 16);
         acc[t] = Ops::pv(a, ph, acc[t]);
+        if constexpr (kP3) acc[t] = Ops::pv(a, pm, acc[t]);
         acc[t] = Ops::pv(a, pl, acc[t]);
       }
     }
