@@ -357,7 +357,7 @@ static int64_t score_slices(int64_t n_samples) {
 // rows: 98 MB) is streamed twice.  Bound by the K stream and by two launches' fixed round
 // trips; a row dot by 16-lane butterflies (six lane exchanges per row and
 // head) had bound it before: 25.1 + 10.4 us for 8 items of 7,564 rows, 4 heads,
-// bf16 D = 128 (15.5 MB), now 6.4 + 7.4 us.
+// bf16 D = 128 (15.5 MB), now 5.9 + 7.8 us.
 template <typename T, int D, bool SCORE>
 __global__ __launch_bounds__(kScoreThreads) void seg_score_kernel(SegScoreParams p) {
   constexpr int EPC = RowGeom<T>::EPC;
